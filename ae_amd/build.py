@@ -19,7 +19,7 @@ CSRC = os.path.join(PKG_DIR, "csrc")
 BUILD_DIR = os.path.join(PKG_DIR, "_build")
 LIB_NAME = "libspecmoe_mi355x.so"
 LIB_PATH = os.path.join(PKG_DIR, LIB_NAME)
-SOURCES = ["routing.hip", "experts.hip", "layer1.hip", "tiles.hip", "capi.hip", "transfer.hip",
+SOURCES = ["routing.hip", "experts.hip", "layer1.hip", "tiles.hip", "wide.hip", "capi.hip", "transfer.hip",
            "stream_probe.hip"]
 ARCH = "gfx950"
 

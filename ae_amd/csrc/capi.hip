@@ -47,6 +47,13 @@ constexpr int64_t kTileLargeTokens = 512;
 // tokens 213.2 vs 213.6; at 64 tokens rows is 1.5-2 us slower (201.4 vs 199.6).
 constexpr int64_t kCombineRowsMinTokens = 128;
 constexpr int64_t kTileMinTokensDefault = 64;
+// Tiled batches of 16-bit types from this many expected tokens per active expert run on the wide
+// tiles (wide.hip, 256 tokens x 256 weight rows) instead of the 128-token tiles: below it their
+// second half is mostly padding and the weights bound the call. Measured per call, 128-token ->
+// wide tiles, at the expected tokens per expert: Mixtral 100: 682 -> 708 us, DeepSeek-V2-Lite 103:
+// 331 -> 369, Qwen1.5-MoE 133: 497 -> 445, Mixtral 175: 822 -> 815, DeepSeek-V2-Lite 192: 490 ->
+// 457, Mixtral 256: 1057 -> 950, 2048: 5705 -> 4850.
+constexpr double kWideMinTokens = 128.0;
 int64_t g_tile_min_tokens = kTileMinTokensDefault;
 // Batches of at most this many tokens run the down projection and the combine as one kernel
 // (down_rows_kernel) instead of the split down kernel plus the combine; negative: the default
@@ -153,6 +160,7 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 
 struct Plan {
   bool tiled = false;  // tiled expert kernels (many tokens per expert) instead of streaming
+  bool wide = false;   // tiled: on the wide tiles
   bool rows = false;   // down projection fused with the combine (a few tokens)
   int N = 0;
   int max_active = 0;  // experts that can be active: min(E, T*k)
@@ -261,12 +269,14 @@ Plan make_plan(int64_t T, int64_t H, int64_t I, int64_t E, int64_t k, int dtype,
   if (p.tiled) {
     p.span = kTileTok;
     p.max_ranges = p.max_active + p.N / p.span;
+    p.wide = eb == 2 && static_cast<double>(p.N) / active >= kWideMinTokens;
+    const int64_t tok = p.wide ? kWideTok : kTileTok;  // tokens of one workgroup's tile
     // K steps of 128 bytes; the down projection's K is split into the fewest parts that give
     // kTileTargetDownBlocks workgroups over the ranges expected
     const int64_t nsteps = I * eb / 128;
-    // ranges expected under uniform routing: each active expert holds ceil(N / active / 128)
+    // tiles of tokens expected under uniform routing: each active expert holds ceil(N / active / tok)
     const int64_t ex = static_cast<int64_t>(active + 0.5);
-    const int64_t per_expert = (static_cast<int64_t>(p.N / active + 0.5) + kTileTok - 1) / kTileTok;
+    const int64_t per_expert = (static_cast<int64_t>(p.N / active + 0.5) + tok - 1) / tok;
     const int64_t ranges = ex * (per_expert < 1 ? 1 : per_expert);
     const int64_t units = ranges * ((H + kTileDownRows - 1) / kTileDownRows);
     const int64_t target = static_cast<double>(p.N) / active >= kTileLargeTokens ? 4 * kTileTargetDownBlocks
@@ -643,8 +653,10 @@ int run_experts(const Plan& p, int dtype, const void* hidden, void* out, int64_t
     mark(4, s);
     return SMX_OK;
   }
-  hipError_t err = p.tiled ? launch_tile_gateup(dtype, a, p.max_ranges, s)
-                           : launch_gateup(dtype, a, p.max_ranges, p.tok_tiles, s, route_g, route_multi, ei);
+  const int pairs = p.max_active + p.N / kWideTok;  // wide tiles: sum of ceil(tokens / kWideTok) at most
+  hipError_t err = p.wide    ? launch_wide(0, dtype, a, pairs, s)
+                   : p.tiled ? launch_tile_gateup(dtype, a, p.max_ranges, s)
+                             : launch_gateup(dtype, a, p.max_ranges, p.tok_tiles, s, route_g, route_multi, ei);
   if (err != hipSuccess) return static_cast<int>(err);
   mark(2, s);
   if (p.rows) {
@@ -675,8 +687,9 @@ int run_experts(const Plan& p, int dtype, const void* hidden, void* out, int64_t
     mark(4, s);  // no combine launch
     return SMX_OK;
   }
-  err = p.tiled ? launch_tile_down(dtype, a, p.max_ranges, s)
-                : launch_down(dtype, a, p.max_ranges, p.tok_tiles, s);
+  err = p.wide    ? launch_wide(1, dtype, a, pairs, s)
+        : p.tiled ? launch_tile_down(dtype, a, p.max_ranges, s)
+                  : launch_down(dtype, a, p.max_ranges, p.tok_tiles, s);
   if (err != hipSuccess) return static_cast<int>(err);
   mark(3, s);
   CombineArgs c{};

@@ -54,6 +54,7 @@ constexpr int kSortRangesMax = kWave + kGateupSortMax / kTokTile;
 constexpr int kTileTok = 128;        // sorted positions per work range
 constexpr int kTileGateCols = 128;   // intermediate columns per gate/up workgroup
 constexpr int kTileDownRows = 256;   // W2 rows per down workgroup
+constexpr int kWideTok = 256;        // tokens of a wide tile (wide.hip): two work ranges
 
 // Work ranges of the expert kernels: up to `span` consecutive sorted positions of one active
 // expert. An expert with more tokens than one pass of the kernels holds is split into nr
@@ -276,6 +277,9 @@ hipError_t launch_combine(int dtype, const CombineArgs& c, hipStream_t s);
 // workgroups, then every work range's weight groups (down: times the K splits).
 int64_t tile_grid_blocks(int stage, int64_t H, int64_t I, int shared_blocks, int max_ranges, int splits);
 hipError_t launch_tile_gateup(int dtype, const ExpertArgs& a, int max_ranges, hipStream_t s);
+// Wide tiles (wide.hip; stage 0: gate/up, 1: down), 16-bit types, span kTileTok: `pairs` bounds the
+// batch's pairs of ranges.
+hipError_t launch_wide(int stage, int dtype, const ExpertArgs& a, int pairs, hipStream_t s);
 hipError_t launch_tile_down(int dtype, const ExpertArgs& a, int max_ranges, hipStream_t s);
 
 }  // namespace smx

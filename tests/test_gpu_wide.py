@@ -1,0 +1,77 @@
+"""GPU parity of the wide tiled kernels (wide.hip: 256 tokens x 256 weight rows, 16-bit types, from
+128 expected tokens per active expert) against the oracle, at the sizes where they can go wrong:
+token counts around the quarters of a tile (64) and around one and two tiles, experts without
+tokens, more pairs of ranges than one wave looks at in one round, several blocks of ranges
+of one expert, H of half a down tile and of one and a half, K walks of two steps, a shared
+expert over several token groups, and routings with dropped assignments."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import moe_ref as ref
+from ae_amd.layers import fused_moe_shared_forward, stack_fused_moe, tiled_min_tokens
+from tests.helpers import TOL, TORCH_TO_ORACLE, f32_of, make_pool, max_rel_err, to_oracle
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _stack(counts, H, I, dtype, seed, unmapped=()):
+    """Every token picks one expert (k = 1): expert e gets counts[e] tokens, in a shuffled order."""
+    E, T = len(counts), sum(counts)
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    ids = torch.repeat_interleave(torch.arange(E, device=DEV), torch.tensor(counts, device=DEV))
+    ids = ids[torch.randperm(T, generator=g, device=DEV)].to(torch.int32).view(T, 1)
+    x = torch.randn((T, H), generator=g, device=DEV).to(dtype)
+    w = torch.rand((T, 1), generator=g, device=DEV) + 0.5
+    pool, slots = make_pool(E, H, I, dtype, num_slots=E + 2, seed=seed + 1)
+    for e in unmapped:
+        slots[e] = -1
+    logits = torch.zeros((T, E), dtype=dtype, device=DEV)
+    with tiled_min_tokens(0):
+        y = stack_fused_moe(x.clone(), pool, slots, logits, w, ids, False, inplace=False)
+    with tiled_min_tokens(1 << 62):
+        ys = stack_fused_moe(x.clone(), pool, slots, logits, w, ids, False, inplace=False)
+    torch.cuda.synchronize()
+    assert torch.isfinite(y.float()).all()
+    # another order of the K sums than the streaming kernels: both lie within TOL of the exact value
+    assert max_rel_err(f32_of(y), f32_of(ys)) <= 2 * TOL[dtype]
+    y_ref = ref.stack_fused_moe(to_oracle(x), to_oracle(pool), slots.cpu().numpy(), w.cpu().numpy(),
+                                ids.cpu().numpy(), TORCH_TO_ORACLE[dtype])
+    assert max_rel_err(f32_of(y), y_ref) <= TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("counts,H,I", [
+    ([1, 511], 128, 128),                       # a one-token tile; two full tiles; two-step walks
+    ([63, 64, 65, 320], 256, 256),
+    ([127, 128, 129, 191, 192, 193], 384, 128),  # one and a half down tiles
+    ([255, 256, 257, 0, 384, 385], 256, 384),
+    ([2049, 0, 1], 128, 256),                   # nine tiles of one expert: three blocks
+    ([200] * 70, 128, 128),                     # 140 ranges, 70 pairs
+])
+def test_wide_token_counts(dtype, counts, H, I):
+    _stack(counts, H, I, dtype, seed=sum(counts) + H)
+
+
+def test_wide_dropped_assignments():
+    _stack([300, 150, 257, 129], 256, 256, torch.bfloat16, seed=7, unmapped=(1,))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,Is", [(257, 640), (1100, 128)])
+def test_wide_shared_expert(dtype, T, Is):
+    H, I, E, k = 256, 128, 4, 2
+    g = torch.Generator(device=DEV).manual_seed(T)
+    x = torch.randn((T, H), generator=g, device=DEV).to(dtype)
+    logits = (torch.randn((T, E), generator=g, device=DEV) * 2.0).to(dtype)
+    sgate = (torch.randn((T, 1), generator=g, device=DEV) * 2.0).to(dtype)
+    page = (torch.randn((3 * Is * H,), generator=g, device=DEV) * 0.02).to(dtype)
+    pool, slots = make_pool(E, H, I, dtype, num_slots=E + 2, seed=E + 1)
+    with tiled_min_tokens(0):
+        y = fused_moe_shared_forward(x.clone(), logits, pool, slots, k, True, page, sgate, 1.0, inplace=False)
+    torch.cuda.synchronize()
+    y_ref, _, _ = ref.fused_moe_shared_forward(
+        to_oracle(x), f32_of(logits), to_oracle(pool), slots.cpu().numpy(), k, True, TORCH_TO_ORACLE[dtype],
+        shared_page=to_oracle(page), shared_gate_logits=f32_of(sgate), routed_scaling_factor=1.0)
+    assert max_rel_err(f32_of(y), y_ref) <= TOL[dtype]
