@@ -229,6 +229,38 @@ int64_t divisor_at_most(int64_t n, int64_t want) {
   return s;
 }
 
+// K splits of the wide down projection: the divisor of its step pairs of the least estimated time,
+// rounds x (steps per split + kWideFixedSteps) x kWideStepUs, one workgroup per CU, plus the bytes
+// the down kernel writes and the combine reads (one split: 16-bit terms; more: fp32 partials).
+// Half a tile of padding is expected per active expert, and half a round of workgroups over what
+// fills the chip (the routing decides the last round). Measured, down + combine in us per call:
+// Mixtral with 1 / 2 / 4 splits, 8192 tokens 1765 / 1823 / 1977, 4096: 974 / 974 / 1082, 2048: 671 /
+// 577 / 588, 1025: 388 / 373 / 359 (before this rule: 4 splits at 2048, 1590 -> 1450 us per call).
+constexpr double kWideStepUs = 1.5;         // one 128-byte K step of a 256 x 256 tile
+constexpr double kWideFixedSteps = 5.0;     // start and end of a workgroup, in steps
+constexpr double kWidePartBytesPerUs = 4.5e6;
+constexpr int64_t kWideMaxSplits = 16;
+int64_t wide_splits(int64_t N, double active, int64_t T, int64_t H, int64_t nsteps, int64_t ssteps, int64_t most) {
+  const int64_t rgroups = (H + kTileDownRows - 1) / kTileDownRows;
+  const double tiles = static_cast<double>(N) / kWideTok + 0.5 * active;
+  const int64_t sgroups = (T + kWideTok - 1) / kWideTok;
+  int64_t best = 1;
+  double best_us = 0.0;
+  for (int64_t s = 1; s <= most && s <= nsteps / 2; ++s) {
+    if ((nsteps / 2) % s != 0) continue;
+    const int64_t per = nsteps / s;
+    const double blocks = rgroups * (tiles * static_cast<double>(s) + static_cast<double>(sgroups * ((ssteps + per - 1) / per)));
+    const double bytes = static_cast<double>(N) * static_cast<double>(H) * (s == 1 ? 4.0 : 8.0 * static_cast<double>(s));
+    const double us = std::max(1.0, blocks / kChipCUs + 0.5) * (static_cast<double>(per) + kWideFixedSteps) * kWideStepUs +
+                      bytes / kWidePartBytesPerUs;
+    if (s == 1 || us < best_us) {
+      best = s;
+      best_us = us;
+    }
+  }
+  return best;
+}
+
 // Limits of the shared expert's intermediate size (the routed limits on I, plus 32-bit
 // offsets into its page and activations).
 int check_shared(int64_t T, int64_t H, int64_t Is, int dtype) {
@@ -270,13 +302,12 @@ Plan make_plan(int64_t T, int64_t H, int64_t I, int64_t E, int64_t k, int dtype,
     p.span = kTileTok;
     p.max_ranges = p.max_active + p.N / p.span;
     p.wide = eb == 2 && static_cast<double>(p.N) / active >= kWideMinTokens;
-    const int64_t tok = p.wide ? kWideTok : kTileTok;  // tokens of one workgroup's tile
     // K steps of 128 bytes; the down projection's K is split into the fewest parts that give
-    // kTileTargetDownBlocks workgroups over the ranges expected
+    // kTileTargetDownBlocks workgroups over the ranges expected (wide tiles: wide_splits)
     const int64_t nsteps = I * eb / 128;
-    // tiles of tokens expected under uniform routing: each active expert holds ceil(N / active / tok)
+    // ranges expected under uniform routing: each active expert holds ceil(N / active / 128)
     const int64_t ex = static_cast<int64_t>(active + 0.5);
-    const int64_t per_expert = (static_cast<int64_t>(p.N / active + 0.5) + tok - 1) / tok;
+    const int64_t per_expert = (static_cast<int64_t>(p.N / active + 0.5) + kTileTok - 1) / kTileTok;
     const int64_t ranges = ex * (per_expert < 1 ? 1 : per_expert);
     const int64_t units = ranges * ((H + kTileDownRows - 1) / kTileDownRows);
     const int64_t target = static_cast<double>(p.N) / active >= kTileLargeTokens ? 4 * kTileTargetDownBlocks
@@ -286,6 +317,13 @@ Plan make_plan(int64_t T, int64_t H, int64_t I, int64_t E, int64_t k, int dtype,
     // split count divides nsteps / 2 (whole: I * eb is a multiple of 256 bytes)
     s = divisor_at_least(nsteps / 2, want);
     if (s > 4 * want) s = divisor_at_most(nsteps / 2, want);
+    if (p.wide) {
+      // a batch whose partials of the 128-token tiles' split count fit the scratch of
+      // smx_fused_moe_forward_noalloc takes at most that many splits: its workspace does not grow
+      const size_t part = sizeof(float) * static_cast<size_t>(s) * static_cast<size_t>(p.N * H);
+      s = wide_splits(p.N, active, T, H, nsteps, Is * eb / 128,
+                      part <= SMX_NOALLOC_SCRATCH_BYTES ? s : kWideMaxSplits);
+    }
     p.splits = static_cast<int>(s);
     p.split_steps = static_cast<int>(nsteps / s * 2);  // in 64-byte units
     if (Is > 0) {
@@ -612,6 +650,8 @@ int run_experts(const Plan& p, int dtype, const void* hidden, void* out, int64_t
   a.k = static_cast<int>(k);
   a.act = b + p.act;
   a.part = reinterpret_cast<float*>(b + p.part);
+  const bool terms = p.wide && p.splits == 1;
+  a.w = terms ? w : nullptr;
   a.splits = p.splits;
   a.split_steps = p.split_steps;
   a.down_rows = p.down_rows;
@@ -707,7 +747,9 @@ int run_experts(const Plan& p, int dtype, const void* hidden, void* out, int64_t
   c.splits_s = p.s_splits;
   c.sgate = bt.sgate;
   c.sgate_dtype = bt.sgate_dtype;
-  c.rows = T >= kCombineRowsMinTokens ? 1 : 0;
+  // (every expert holds at most T tokens: a wide batch has kWideMinTokens or more)
+  c.rows = T >= kCombineRowsMinTokens || terms ? 1 : 0;
+  c.terms = terms ? 1 : 0;
   c.f16out = a.f16out;
   err = launch_combine(dtype, c, s);
   if (err != hipSuccess) return static_cast<int>(err);

@@ -224,7 +224,9 @@ constexpr int kCombineRowThreads = 256;
 constexpr int kCombineRowOuts = 8;
 constexpr int kCombineRowBatch = 8;  // assignments whose partials are loaded together
 
-template <int DT>
+// kTerms: one split whose terms round(w * sum) the down kernel has written in the activation type
+// (CombineArgs::terms): they are only added, in the same order (the same bits).
+template <int DT, bool kTerms = false>
 __global__ __launch_bounds__(kCombineRowThreads) void combine_rows_kernel(CombineArgs c) {
   // thread g owns outputs [8g, 8g + 8): token g / (H/8); T*H/8 < 2^31 (one chunk of the call)
   const int per_t = c.H / kCombineRowOuts;
@@ -242,8 +244,9 @@ __global__ __launch_bounds__(kCombineRowThreads) void combine_rows_kernel(Combin
   const bool gated = shared && c.sgate != nullptr;
   const float zs = gated ? load_scalar(c.sgate, c.sgate_dtype, t) : 0.0f;
   const int64_t sstride = static_cast<int64_t>(c.T) * c.H;
+  // (the terms take half the bytes of `part`: its row t * k / 2 is the token's first)
   const float* ssrc = shared ? c.part_s + static_cast<int64_t>(t) * c.H + h
-                             : c.part + static_cast<int64_t>(t) * c.k * c.H + h;
+                             : c.part + static_cast<int64_t>(kTerms ? t * c.k / 2 : t * c.k) * c.H + h;
   const int64_t s1 = shared && c.splits_s > 1 ? sstride : 0;
   const f32x4 ps0a = *reinterpret_cast<const f32x4*>(ssrc);
   const f32x4 ps0b = *reinterpret_cast<const f32x4*>(ssrc + 4);
@@ -254,7 +257,26 @@ __global__ __launch_bounds__(kCombineRowThreads) void combine_rows_kernel(Combin
   // kCombineRowBatch assignments at a time: their weights and partials (from clamped j, in
   // bounds: every row f = t*k + j of part exists) are loaded together, then summed over the
   // splits in split order and added over j in order -- the arithmetic of combine_kernel.
-  for (int j0 = 0; j0 < c.k; j0 += kCombineRowBatch) {
+  for (int j0 = 0; kTerms && j0 < c.k; j0 += kCombineRowBatch) {
+    using S = typename Elem<DT>::S;
+    const S* src0 = reinterpret_cast<const S*>(c.part) + static_cast<int64_t>(t) * c.k * c.H + h;
+    u32x4 v[kCombineRowBatch];
+#pragma unroll
+    for (int jj = 0; jj < kCombineRowBatch; ++jj)
+      v[jj] = *reinterpret_cast<const u32x4*>(src0 + static_cast<int64_t>(min(j0 + jj, c.k - 1)) * c.H);
+#pragma unroll
+    for (int jj = 0; jj < kCombineRowBatch; ++jj) {
+      const int j = j0 + jj;
+      if (j < c.k && ((vm >> j) & 1u)) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          y0[e] += Elem<DT>::to_f32(static_cast<S>(v[jj][e / 2] >> (16 * (e % 2))));
+          y1[e] += Elem<DT>::to_f32(static_cast<S>(v[jj][2 + e / 2] >> (16 * (e % 2))));
+        }
+      }
+    }
+  }
+  for (int j0 = 0; !kTerms && j0 < c.k; j0 += kCombineRowBatch) {
     const float* src0 = c.part + (static_cast<int64_t>(t) * c.k) * c.H + h;
     float wf[kCombineRowBatch];
     f32x4 v0[kCombineRowBatch], v1[kCombineRowBatch];
@@ -704,8 +726,14 @@ hipError_t launch_combine(int dtype, const CombineArgs& c, hipStream_t s) {
     const unsigned blocks = static_cast<unsigned>((outs + threads - 1) / threads);
     switch (dtype) {
       case kF32: combine_rows_kernel<kF32><<<blocks, threads, 0, s>>>(c); break;
-      case kF16: combine_rows_kernel<kF16><<<blocks, threads, 0, s>>>(c); break;
-      default: combine_rows_kernel<kBF16><<<blocks, threads, 0, s>>>(c); break;
+      case kF16:
+        if (c.terms) combine_rows_kernel<kF16, true><<<blocks, threads, 0, s>>>(c);
+        else combine_rows_kernel<kF16><<<blocks, threads, 0, s>>>(c);
+        break;
+      default:
+        if (c.terms) combine_rows_kernel<kBF16, true><<<blocks, threads, 0, s>>>(c);
+        else combine_rows_kernel<kBF16><<<blocks, threads, 0, s>>>(c);
+        break;
     }
     return hipGetLastError();
   }

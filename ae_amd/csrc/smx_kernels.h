@@ -146,6 +146,8 @@ struct ExpertArgs {
   int T, H, I, k;
   void* act;            // [T*k, I] silu(gate)*up, row = sorted position
   float* part;          // [splits, T*k, H] fp32 partial down projections, row = f
+  const float* w;       // [T*k] routing weights when the wide down kernel writes finished terms into
+                        // `part` (CombineArgs::terms), null when it writes fp32 partials
   int splits;           // K splits of the down projection
   int split_steps;      // load steps per split
   int f16out;           // fp32 runs: routed gate/up outputs rounded to fp16 (reference stores)
@@ -178,6 +180,8 @@ struct CombineArgs {
   int sgate_dtype;
   int rows;                  // thread-per-outputs kernel (large batches) instead of per-token
   int f16out;                // fp32 runs: each routed term rounded to fp16 (reference stores)
+  int terms;                 // rows kernel, 16-bit types: `part` holds the finished terms
+                             // round(w * sum) [T*k, H] in the activation type (one split)
 };
 
 // Down projection fused with the combine for batches of a few tokens (experts.hip,

@@ -353,6 +353,18 @@ __device__ __forceinline__ float silu_rcp(float g) {
   return g > 100.0f ? g : q;  // 1 + e^-g is 1; keeps +inf (whose hi + lo is NaN)
 }
 
+// Rows of 16 lanes hold 4 consecutive columns each of two 16-column tiles of one output row: `a`
+// (tile 0) and `b` (tile 1), packed. Swapping a's odd rows with b's even ones leaves 8 consecutive
+// columns in every lane -- of tile g % 2, from column 8 (g / 2), g the row -- so that a store
+// writes 16 bytes per lane and 64 contiguous bytes per output row instead of 8 and 32.
+__device__ __forceinline__ u32x4 join_tiles(const u32x2& a, const u32x2& b) {
+  const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false));
+  const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false));
+  return u32x4{lo[0], hi[0], lo[1], hi[1]};
+}
+// The lane's first column of a joined pair of tiles.
+__device__ __forceinline__ int join_col(int lane) { return ((lane >> 4) & 1) * kRowTile + (lane >> 5) * 8; }
+
 struct WideStages {
   u32x4 *a0, *b0, *a1, *b1;
 };
@@ -366,45 +378,76 @@ __device__ __forceinline__ void wide_gateup_item(const ExpertArgs& a, const Work
   wide_walk<DT, NT>(src, st.a0, st.b0, st.a1, st.b1, ln, acc);
   S* act = static_cast<S*>(it.shared ? a.sh.act : a.act);
   const int lane = lane_id();
-  const int col0 = it.tg * kTileGateCols + ln.wr * (kXTiles / 2) * kRowTile + 4 * (lane >> 4);
+  const int col0 = it.tg * kTileGateCols + ln.wr * (kXTiles / 2) * kRowTile + join_col(lane);
 #pragma unroll
   for (int j = 0; j < NT; ++j) {
     const int q = (ln.wt + kXTokGroups * j) * kTokTile + (lane & 15);
-    if (q >= it.m) continue;
+    if (q >= it.m) continue;  // the same for the four lanes of an output row
     const int64_t row = static_cast<int64_t>(it.off + q) * it.I + col0;
 #pragma unroll
-    for (int i = 0; i < kXTiles / 2; ++i) {
-      const f32x4 gacc = acc[i][j], uacc = acc[i + kXTiles / 2][j];
-      u32x2 v;
+    for (int i = 0; i < kXTiles / 2; i += 2) {
+      u32x2 v[2];
 #pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        const f32x2 gate = unpack2<DT>(pack2<DT>(gacc[2 * e], gacc[2 * e + 1]));
-        const f32x2 up = unpack2<DT>(pack2<DT>(uacc[2 * e], uacc[2 * e + 1]));
-        v[e] = pack2<DT>(silu_rcp(gate[0]) * up[0], silu_rcp(gate[1]) * up[1]);
+      for (int p = 0; p < 2; ++p) {
+        const f32x4 gacc = acc[i + p][j], uacc = acc[i + p + kXTiles / 2][j];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const f32x2 gate = unpack2<DT>(pack2<DT>(gacc[2 * e], gacc[2 * e + 1]));
+          const f32x2 up = unpack2<DT>(pack2<DT>(uacc[2 * e], uacc[2 * e + 1]));
+          v[p][e] = pack2<DT>(silu_rcp(gate[0]) * up[0], silu_rcp(gate[1]) * up[1]);
+        }
       }
-      *reinterpret_cast<u32x2*>(act + row + i * kRowTile) = v;
+      *reinterpret_cast<u32x4*>(act + row + i * kRowTile) = join_tiles(v[0], v[1]);
     }
   }
 }
 
-template <int DT, int NT>
+template <int DT, int NT, bool kTerms>
 __device__ __forceinline__ void wide_down_item(const ExpertArgs& a, const WorkItem& it, int sp, int h0, int rows,
                                                const WideSrc& src, const WideStages& st, const WideLane& ln) {
+  using S = typename Elem<DT>::S;
+  const int lane = lane_id();
+  // the rows' assignments and weights, loaded before the walk: their two latencies pass under it
+  int fs[NT];
+  float ws[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j) {
+    const int q = it.off + min((ln.wt + kXTokGroups * j) * kTokTile + (lane & 15), it.m - 1);
+    fs[j] = it.shared ? q : a.rb.sorted_f[q];
+  }
+#pragma unroll
+  for (int j = 0; j < NT; ++j) ws[j] = kTerms ? a.w[fs[j]] : 0.0f;
   f32x4 acc[kXTiles][NT];
   wide_zero<NT>(acc);
   wide_walk<DT, NT>(src, st.a0, st.b0, st.a1, st.b1, ln, acc);
   float* part = it.shared ? a.sh.part : a.part;
-  const int lane = lane_id();
 #pragma unroll
   for (int j = 0; j < NT; ++j) {
     const int q = (ln.wt + kXTokGroups * j) * kTokTile + (lane & 15);
     if (q >= it.m) continue;
-    const int f = it.shared ? it.off + q : a.rb.sorted_f[it.off + q];
-    float* dst = part + (static_cast<int64_t>(sp) * rows + f) * a.H;
+    const int f = fs[j];
+    if constexpr (kTerms) {
+      const float wf = ws[j];
+      S* dst = reinterpret_cast<S*>(part) + static_cast<int64_t>(f) * a.H + join_col(lane);
 #pragma unroll
-    for (int i = 0; i < kXTiles; ++i) {
-      const int h = h0 + wide_a_slot(i) / kXSlots + ln.wr * (kXTiles / 2) * kRowTile;
-      if (h < a.H) *reinterpret_cast<f32x4*>(dst + h + 4 * (lane >> 4)) = acc[i][j];
+      for (int i = 0; i < kXTiles; i += 2) {
+        const int h = h0 + wide_a_slot(i) / kXSlots + ln.wr * (kXTiles / 2) * kRowTile;
+        u32x2 v[2];
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          const f32x4 d = acc[i + p][j];
+          v[p] = u32x2{pack2<DT>(d[0] * wf, d[1] * wf), pack2<DT>(d[2] * wf, d[3] * wf)};
+        }
+        const u32x4 o = join_tiles(v[0], v[1]);
+        if (h < a.H) *reinterpret_cast<u32x4*>(dst + h) = o;
+      }
+    } else {
+      float* dst = part + (static_cast<int64_t>(sp) * rows + f) * a.H + 4 * (lane >> 4);
+#pragma unroll
+      for (int i = 0; i < kXTiles; ++i) {
+        const int h = h0 + wide_a_slot(i) / kXSlots + ln.wr * (kXTiles / 2) * kRowTile;
+        if (h < a.H) *reinterpret_cast<f32x4*>(dst + h) = acc[i][j];
+      }
     }
   }
 }
@@ -456,8 +499,12 @@ __global__ __launch_bounds__(kXThreads, 1) void wide_gateup_kernel(ExpertArgs a)
 }
 
 // Workgroup = (pair of token ranges, 256 rows of W2, K split): fp32 partials part[split][f][h],
-// summed by the combine. Rows past H (a multiple of 128) are clamped and not stored.
-template <int DT>
+// summed by the combine; with one split the routed sums are whole, and the kernel rounds them
+// times their routing weight (the combine's own rounding) and writes these terms at half the
+// bytes, which the combine only adds (per call, fp32 partials -> terms, down + combine:
+// DeepSeek-V2-Lite 2047 tokens 159 + 31 -> 153 + 20 us, Mixtral 8192 tokens 1742 + 122 -> 1716 +
+// 48). Rows past H (a multiple of 128) are clamped and not stored.
+template <int DT, bool kTerms>
 __global__ __launch_bounds__(kXThreads, 1) void wide_down_kernel(ExpertArgs a) {
   using S = typename Elem<DT>::S;
   const int rgroups = (a.H + kTileDownRows - 1) / kTileDownRows;
@@ -490,11 +537,20 @@ __global__ __launch_bounds__(kXThreads, 1) void wide_down_kernel(ExpertArgs a) {
   src.n = split_steps * kStepBytes / kXStep;
   src.rot = wide_rot(it.rot, src.n);
   const WideStages st{a0, b0, a1, b1};
-  switch (wide_quarters(it.m)) {
-    case 1: wide_down_item<DT, 2>(a, it, sp, h0, rows, src, st, ln); break;
-    case 2: wide_down_item<DT, 4>(a, it, sp, h0, rows, src, st, ln); break;
-    case 3: wide_down_item<DT, 6>(a, it, sp, h0, rows, src, st, ln); break;
-    default: wide_down_item<DT, 8>(a, it, sp, h0, rows, src, st, ln); break;
+  auto item = [&](auto terms) {
+    constexpr bool kT = decltype(terms)::value;
+    switch (wide_quarters(it.m)) {
+      case 1: wide_down_item<DT, 2, kT>(a, it, sp, h0, rows, src, st, ln); break;
+      case 2: wide_down_item<DT, 4, kT>(a, it, sp, h0, rows, src, st, ln); break;
+      case 3: wide_down_item<DT, 6, kT>(a, it, sp, h0, rows, src, st, ln); break;
+      default: wide_down_item<DT, 8, kT>(a, it, sp, h0, rows, src, st, ln); break;
+    }
+  };
+  if constexpr (kTerms) {
+    if (!it.shared) item(std::true_type{});
+    else item(std::false_type{});
+  } else {
+    item(std::false_type{});
   }
   wide_drain();
 }
@@ -519,7 +575,10 @@ static hipError_t wide_launch(int stage, ExpertArgs a, int pairs, hipStream_t s)
       return hipErrorInvalidValue;
     a.sh.down_blocks = sgroups * rgroups * a.sh.splits;
     const int64_t blocks = a.sh.down_blocks + static_cast<int64_t>(pairs) * rgroups * a.splits;
-    wide_down_kernel<DT><<<static_cast<unsigned>(blocks), kXThreads, 0, s>>>(a);
+    if (a.w != nullptr && a.splits == 1)
+      wide_down_kernel<DT, true><<<static_cast<unsigned>(blocks), kXThreads, 0, s>>>(a);
+    else
+      wide_down_kernel<DT, false><<<static_cast<unsigned>(blocks), kXThreads, 0, s>>>(a);
   }
   return hipGetLastError();
 }
