@@ -568,12 +568,15 @@ __global__ __launch_bounds__(kWave) void route_small_kernel(
 // specmoe/models/mixtral.py:310-313.
 // ---------------------------------------------------------------------------------------
 // RB = router rows per batch (8, 16 or 32).
-template <int DT, int G, int PL, int RB>
+// kDyn: the token's row in dynamic LDS (H floats).
+template <int DT, int G, int PL, int RB, bool kDyn>
 __global__ __launch_bounds__(kNormThreads) void norm_gate_kernel(NormGateArgs a) {
   static_assert(RB == 8 || RB == 16 || RB == 32, "P = 256 / RB lanes reduce a row");
   using S = typename Elem<DT>::S;
   constexpr int V = 16 / static_cast<int>(sizeof(S));  // elements per 16-byte vector
-  __shared__ float sb[kNormMaxH];
+  extern __shared__ __align__(16) float dyn_row[];
+  __shared__ float fixed_row[kDyn ? 4 : kNormMaxH];
+  float* const sb = kDyn ? dyn_row : fixed_row;
   __shared__ float red[kNormWaves];
   __shared__ float lg[kMaxExperts];
   const int t = blockIdx.x;
@@ -915,7 +918,14 @@ hipError_t launch_route(const void* logits, int ldt, int T, int E, int k, int re
 
 template <int DT, int G, int PL, int RB>
 static void norm_gate_launch(const NormGateArgs& a, hipStream_t s) {
-  norm_gate_kernel<DT, G, PL, RB><<<a.T, kNormThreads, 0, s>>>(a);
+  // LDS for the token's row only, so that a CU holds as many workgroups as that leaves room for --
+  // two with the largest row's fixed 64 KB, too few to cover the gate rows' L2 latency
+  // (DeepSeek-V2-Lite layer of 2047 tokens 483.6 -> 475.8 us). A batch that two workgroups per CU
+  // hold keeps the fixed row (32 tokens 187.1 us against 188.2).
+  if (a.T > 2 * kNormCUs)
+    norm_gate_kernel<DT, G, PL, RB, true><<<a.T, kNormThreads, sizeof(float) * a.H, s>>>(a);
+  else
+    norm_gate_kernel<DT, G, PL, RB, false><<<a.T, kNormThreads, 0, s>>>(a);
 }
 
 // Top-k lane groups from E; router rows per batch from the row count (E + shared-gate row).

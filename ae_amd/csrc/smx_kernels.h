@@ -230,6 +230,7 @@ hipError_t launch_layer1(int dtype, const ExpertArgs& a, int max_ranges, int rou
 // Post-attention residual add + RMSNorm + router gate (+ shared-expert gate row, + top-k).
 constexpr int kNormThreads = 256;
 constexpr int kNormWaves = kNormThreads / kWave;
+constexpr int kNormCUs = 256;     // compute units of the chip
 constexpr int kNormMaxH = 16384;  // one token's fp32 row is staged in LDS
 
 struct NormGateArgs {
