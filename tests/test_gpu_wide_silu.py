@@ -1,6 +1,7 @@
 """SiLU of the wide tiled kernels (wide.hip) at every value a 16-bit gate can take: the class (finite,
-infinite, NaN), in bf16 the bits of the weight-streaming kernels' outputs, and the exact value
-rounded to the activation type. One expert; each token carries one gate pattern.
+infinite, NaN) and the bits of the weight-streaming kernels' outputs, and the exact value rounded
+to the activation type; and the bits of the terms that the down projection weighs. One expert;
+each token carries one gate pattern.
 
 The finite gates: x[t] = (pattern_t, 1, 0, ...), W1 row i = (1, 0, ...), W3 row i = (0, u_i, 0, ...),
 W2 = identity: output h is round(silu(pattern_t) * u_h), with no sum of more than one non-zero
@@ -19,11 +20,11 @@ H = I = 128
 FORM = {torch.bfloat16: (7, -126), torch.float16: (10, -14)}
 
 
-def _layer(x, w1, w3, w2, wide):
+def _layer(x, w1, w3, w2, wide, w=None):
     T = x.shape[0]
     pool = torch.cat([w1.reshape(-1), w3.reshape(-1), w2.reshape(-1)]).to(x.dtype).view(1, -1)
     ids = torch.zeros((T, 1), dtype=torch.int32, device=DEV)
-    w = torch.ones((T, 1), device=DEV)
+    w = torch.ones((T, 1), device=DEV) if w is None else w
     slots = torch.zeros((1,), dtype=torch.int64, device=DEV)
     logits = torch.zeros((T, 1), dtype=x.dtype, device=DEV)
     with tiled_min_tokens(0 if wide else 1 << 62):
@@ -32,8 +33,7 @@ def _layer(x, w1, w3, w2, wide):
     return y
 
 
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-def test_every_finite_gate(dtype):
+def _finite_gates(dtype):
     p = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(dtype)
     p = p[torch.isfinite(p.float())].to(DEV)
     u = (0.5 + torch.arange(I, device=DEV) / (2.0 * I)).to(dtype)  # exact in both types
@@ -43,12 +43,16 @@ def test_every_finite_gate(dtype):
     w1[:, 0] = 1.0
     w3 = torch.zeros((I, H), device=DEV)
     w3[:, 1] = u.float()
-    w2 = torch.eye(H, I, device=DEV)
+    return p, u, x, w1, w3, torch.eye(H, I, device=DEV)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_every_finite_gate(dtype):
+    p, u, x, w1, w3, w2 = _finite_gates(dtype)
     y = _layer(x, w1, w3, w2, True)
     assert torch.isfinite(y.float()).all(), int((~torch.isfinite(y.float())).any(1).sum())
     ys = _layer(x, w1, w3, w2, False)
-    if dtype == torch.bfloat16:
-        assert torch.equal(y.view(torch.int16), ys.view(torch.int16))
+    assert torch.equal(y.view(torch.int16), ys.view(torch.int16))
     g = p.double()
     exact = (g / (1.0 + torch.exp(-g)))[:, None] * u.double()
     # half a unit of the type for its rounding; the fp32 value before it is within 2^-21 of the
@@ -63,6 +67,16 @@ def test_every_finite_gate(dtype):
     assert (err <= (0.5 + 2.0 ** -9) * unit)[~small & ~over].all(), (err / unit)[~small & ~over].max().item()
     assert (err <= 2.0 ** emin)[small].all()
     assert (y[over] == 0).all() and (exact[over] >= -2.8e-37).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_weighted_terms(dtype):
+    """One K split: the down kernel rounds weight * sum itself, as the combine does elsewhere."""
+    p, _, x, w1, w3, w2 = _finite_gates(dtype)
+    g = torch.Generator(device=DEV).manual_seed(5)
+    w = torch.rand((p.numel(), 1), generator=g, device=DEV) + 0.25
+    y, ys = (_layer(x, w1, w3, w2, wide, w) for wide in (True, False))
+    assert torch.equal(y.view(torch.int16), ys.view(torch.int16))
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
