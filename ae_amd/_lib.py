@@ -141,7 +141,7 @@ PLAN_FIELDS = ("tiled", "fused_down", "span", "max_ranges", "tok_tiles", "splits
                "shared_split_steps", "shared_tok_groups", "shared_gateup_blocks",
                "shared_down_blocks", "tile_gateup_grid", "tile_down_grid", "single_launch",
                "sync_blocks", "sync_offset", "topk_in_gateup", "expert_items", "chunk_tokens",
-               "workspace_bytes")
+               "workspace_bytes", "wide_pairs")
 
 
 def plan_info(T: int, H: int, I: int, E: int, top_k: int, dtype: int, shared_I: int = 0) -> dict:

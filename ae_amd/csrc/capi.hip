@@ -160,7 +160,7 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 
 struct Plan {
   bool tiled = false;  // tiled expert kernels (many tokens per expert) instead of streaming
-  bool wide = false;   // tiled: on the wide tiles
+  int wide_pairs = 0;  // tiled: on the wide tiles, with grids for this many pairs of ranges (0: not)
   bool rows = false;   // down projection fused with the combine (a few tokens)
   int N = 0;
   int max_active = 0;  // experts that can be active: min(E, T*k)
@@ -301,7 +301,8 @@ Plan make_plan(int64_t T, int64_t H, int64_t I, int64_t E, int64_t k, int dtype,
   if (p.tiled) {
     p.span = kTileTok;
     p.max_ranges = p.max_active + p.N / p.span;
-    p.wide = eb == 2 && static_cast<double>(p.N) / active >= kWideMinTokens;
+    const bool wide = eb == 2 && static_cast<double>(p.N) / active >= kWideMinTokens;
+    if (wide) p.wide_pairs = p.max_active + p.N / kWideTok;  // sum of ceil(tokens / kWideTok) at most
     // K steps of 128 bytes; the down projection's K is split into the fewest parts that give
     // kTileTargetDownBlocks workgroups over the ranges expected (wide tiles: wide_splits)
     const int64_t nsteps = I * eb / 128;
@@ -317,7 +318,7 @@ Plan make_plan(int64_t T, int64_t H, int64_t I, int64_t E, int64_t k, int dtype,
     // split count divides nsteps / 2 (whole: I * eb is a multiple of 256 bytes)
     s = divisor_at_least(nsteps / 2, want);
     if (s > 4 * want) s = divisor_at_most(nsteps / 2, want);
-    if (p.wide) {
+    if (wide) {
       // a batch whose partials of the 128-token tiles' split count fit the scratch of
       // smx_fused_moe_forward_noalloc takes at most that many splits: its workspace does not grow
       const size_t part = sizeof(float) * static_cast<size_t>(s) * static_cast<size_t>(p.N * H);
@@ -333,7 +334,8 @@ Plan make_plan(int64_t T, int64_t H, int64_t I, int64_t E, int64_t k, int dtype,
       p.Is = static_cast<int>(Is);
       p.s_splits = static_cast<int>(ss);
       p.s_split_steps = static_cast<int>(ssteps / ss * 2);
-      p.s_tok_groups = static_cast<int>((T + p.span - 1) / p.span);
+      const int tok = wide ? kWideTok : p.span;
+      p.s_tok_groups = static_cast<int>((T + tok - 1) / tok);
       p.s_gateup_blocks = static_cast<int>(p.s_tok_groups * ((Is + kTileGateCols - 1) / kTileGateCols));
       p.s_down_blocks = static_cast<int>(p.s_tok_groups * ((H + kTileDownRows - 1) / kTileDownRows) * ss);
     }
@@ -650,7 +652,7 @@ int run_experts(const Plan& p, int dtype, const void* hidden, void* out, int64_t
   a.k = static_cast<int>(k);
   a.act = b + p.act;
   a.part = reinterpret_cast<float*>(b + p.part);
-  const bool terms = p.wide && p.splits == 1;
+  const bool terms = p.wide_pairs > 0 && p.splits == 1;
   a.w = terms ? w : nullptr;
   a.splits = p.splits;
   a.split_steps = p.split_steps;
@@ -693,10 +695,9 @@ int run_experts(const Plan& p, int dtype, const void* hidden, void* out, int64_t
     mark(4, s);
     return SMX_OK;
   }
-  const int pairs = p.max_active + p.N / kWideTok;  // wide tiles: sum of ceil(tokens / kWideTok) at most
-  hipError_t err = p.wide    ? launch_wide(0, dtype, a, pairs, s)
-                   : p.tiled ? launch_tile_gateup(dtype, a, p.max_ranges, s)
-                             : launch_gateup(dtype, a, p.max_ranges, p.tok_tiles, s, route_g, route_multi, ei);
+  hipError_t err = p.wide_pairs > 0 ? launch_wide(0, dtype, a, p.wide_pairs, s)
+                   : p.tiled        ? launch_tile_gateup(dtype, a, p.max_ranges, s)
+                                    : launch_gateup(dtype, a, p.max_ranges, p.tok_tiles, s, route_g, route_multi, ei);
   if (err != hipSuccess) return static_cast<int>(err);
   mark(2, s);
   if (p.rows) {
@@ -727,9 +728,9 @@ int run_experts(const Plan& p, int dtype, const void* hidden, void* out, int64_t
     mark(4, s);  // no combine launch
     return SMX_OK;
   }
-  err = p.wide    ? launch_wide(1, dtype, a, pairs, s)
-        : p.tiled ? launch_tile_down(dtype, a, p.max_ranges, s)
-                  : launch_down(dtype, a, p.max_ranges, p.tok_tiles, s);
+  err = p.wide_pairs > 0 ? launch_wide(1, dtype, a, p.wide_pairs, s)
+        : p.tiled        ? launch_tile_down(dtype, a, p.max_ranges, s)
+                         : launch_down(dtype, a, p.max_ranges, p.tok_tiles, s);
   if (err != hipSuccess) return static_cast<int>(err);
   mark(3, s);
   CombineArgs c{};
@@ -936,8 +937,9 @@ int smx_moe_plan_info(int64_t T, int64_t H, int64_t I, int64_t E, int64_t top_k,
   v[SMX_PLAN_SHARED_GATEUP_BLOCKS] = p.s_gateup_blocks;
   v[SMX_PLAN_SHARED_DOWN_BLOCKS] = p.s_down_blocks;
   if (p.tiled) {
-    v[SMX_PLAN_TILE_GATEUP_GRID] = tile_grid_blocks(0, H, I, p.s_gateup_blocks, p.max_ranges, 1);
-    v[SMX_PLAN_TILE_DOWN_GRID] = tile_grid_blocks(1, H, I, p.s_down_blocks, p.max_ranges, p.splits);
+    const int items = p.wide_pairs > 0 ? p.wide_pairs : p.max_ranges;
+    v[SMX_PLAN_TILE_GATEUP_GRID] = tile_grid_blocks(0, H, I, p.s_gateup_blocks, items, 1);
+    v[SMX_PLAN_TILE_DOWN_GRID] = tile_grid_blocks(1, H, I, p.s_down_blocks, items, p.splits);
   }
   v[SMX_PLAN_SINGLE_LAUNCH] = p.layer1 && g_layer1;
   v[SMX_PLAN_SYNC_BLOCKS] = p.layer1 ? p.sync_blocks : 0;
@@ -949,6 +951,7 @@ int smx_moe_plan_info(int64_t T, int64_t H, int64_t I, int64_t E, int64_t top_k,
   v[SMX_PLAN_EXPERT_ITEMS] = ids_multi && expert_items_apply(p, Tp, E, top_k);
   v[SMX_PLAN_CHUNK_TOKENS] = tc;
   v[SMX_PLAN_WORKSPACE_BYTES] = static_cast<int64_t>(workspace_for(T, H, I, E, top_k, dtype, shared_I, false));
+  v[SMX_PLAN_WIDE_PAIRS] = p.wide_pairs;
   for (int i = 0; i < n && i < SMX_PLAN_FIELDS; ++i) out[i] = v[i];
   return SMX_PLAN_FIELDS;
 }

@@ -283,7 +283,7 @@ hipError_t launch_combine(int dtype, const CombineArgs& c, hipStream_t s);
 int64_t tile_grid_blocks(int stage, int64_t H, int64_t I, int shared_blocks, int max_ranges, int splits);
 hipError_t launch_tile_gateup(int dtype, const ExpertArgs& a, int max_ranges, hipStream_t s);
 // Wide tiles (wide.hip; stage 0: gate/up, 1: down), 16-bit types, span kTileTok: `pairs` bounds the
-// batch's pairs of ranges.
+// batch's pairs of ranges (the grid: tile_grid_blocks of them), sh.tok_groups counts kWideTok tokens.
 hipError_t launch_wide(int stage, int dtype, const ExpertArgs& a, int pairs, hipStream_t s);
 hipError_t launch_tile_down(int dtype, const ExpertArgs& a, int max_ranges, hipStream_t s);
 

@@ -238,7 +238,7 @@ __device__ __forceinline__ bool wide_item(const ExpertArgs& a, int shared_blocks
   const int b = static_cast<int>(blockIdx.x);
   int r, g;
   if (b < shared_blocks) {
-    const int nr = (a.T + kWideTok - 1) / kWideTok;
+    const int nr = a.sh.tok_groups;
     wide_range_group(b, per_item, nr, r, g);
     w.page = static_cast<const char*>(a.sh.page);
     w.page_bytes = 3 * static_cast<int64_t>(a.H) * a.sh.I * elem;
@@ -564,26 +564,21 @@ __global__ __launch_bounds__(kXThreads, 1) void wide_down_kernel(ExpertArgs a) {
   wide_drain();
 }
 
-// `a` with the shared expert's leading workgroups of the wide tiles; pairs: routed pairs at most.
 template <int DT>
-static hipError_t wide_launch(int stage, ExpertArgs a, int pairs, hipStream_t s) {
-  const int sgroups = a.sh.I > 0 ? (a.T + kWideTok - 1) / kWideTok : 0;
-  const int rgroups = (a.H + kTileDownRows - 1) / kTileDownRows;
+static hipError_t wide_launch(int stage, const ExpertArgs& a, int pairs, hipStream_t s) {
   const int64_t eb = dtype_bytes(DT);
   // the walk consumes K steps in pairs, and the tiles cover whole 128-column groups: the plan
   // gives both (H and I are whole 256-byte chunks, split counts divide half the steps)
   auto odd = [](int64_t bytes) { return bytes <= 0 || bytes % (2 * kXStep) != 0; };
   if (stage == 0) {
     if (odd(a.H * eb) || a.I % kTileGateCols != 0 || a.sh.I % kTileGateCols != 0) return hipErrorInvalidValue;
-    a.sh.gateup_blocks = sgroups * (a.sh.I / kTileGateCols);
-    const int64_t blocks = a.sh.gateup_blocks + static_cast<int64_t>(pairs) * (a.I / kTileGateCols);
+    const int64_t blocks = tile_grid_blocks(0, a.H, a.I, a.sh.gateup_blocks, pairs, 1);
     wide_gateup_kernel<DT><<<static_cast<unsigned>(blocks), kXThreads, 0, s>>>(a);
   } else {
     if (odd(static_cast<int64_t>(a.split_steps) * kStepBytes) ||
         (a.sh.I > 0 && odd(static_cast<int64_t>(a.sh.split_steps) * kStepBytes)))
       return hipErrorInvalidValue;
-    a.sh.down_blocks = sgroups * rgroups * a.sh.splits;
-    const int64_t blocks = a.sh.down_blocks + static_cast<int64_t>(pairs) * rgroups * a.splits;
+    const int64_t blocks = tile_grid_blocks(1, a.H, a.I, a.sh.down_blocks, pairs, a.splits);
     if (a.w != nullptr && a.splits == 1)
       wide_down_kernel<DT, true><<<static_cast<unsigned>(blocks), kXThreads, 0, s>>>(a);
     else

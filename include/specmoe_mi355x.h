@@ -316,7 +316,8 @@ int smx_h2d_pending(smx_h2d_engine* engine);
  * Expert-kernel selection. A MoE call whose expected tokens per active expert -- T*top_k
  * divided by the experts expected to be active under uniform routing,
  * E*(1 - (1 - top_k/E)^T) -- is at least `tokens_per_expert` runs the tiled expert kernels
- * (MFMA output tiles of 128 tokens by 128 intermediate columns / 256 hidden rows, for
+ * (MFMA output tiles of 128 intermediate columns / 256 hidden rows by 128 tokens, or by 256 tokens
+ * for bf16 and fp16 batches of hundreds of tokens per expert (SMX_PLAN_WIDE_PAIRS); for
  * prefill-sized batches); below it, the weight-streaming kernels. 0 = always tiled,
  * INT64_MAX = never; a negative value restores the default (64). Both produce the same
  * routing and rounding points; only the fp32 summation order over K differs. The workspace
@@ -464,7 +465,8 @@ enum smx_plan_field {
   SMX_PLAN_TILED = 0,           /* 1: tiled MFMA expert kernels; 0: weight-streaming kernels */
   SMX_PLAN_FUSED_DOWN,          /* 1: down projection fused with the combine (few tokens) */
   SMX_PLAN_SPAN,                /* sorted positions per work range */
-  SMX_PLAN_MAX_RANGES,          /* work ranges the grids are sized for */
+  SMX_PLAN_MAX_RANGES,          /* work ranges at most (the grids are sized for them, or for
+                                   SMX_PLAN_WIDE_PAIRS) */
   SMX_PLAN_TOK_TILES,           /* 16-token tiles per range (streaming kernels) */
   SMX_PLAN_SPLITS,              /* K splits of the routed down projection */
   SMX_PLAN_SPLIT_STEPS,         /* 64-byte steps per down split */
@@ -491,6 +493,8 @@ enum smx_plan_field {
                                    by expert (smx_set_gateup_expert_items) */
   SMX_PLAN_CHUNK_TOKENS,        /* tokens per pass */
   SMX_PLAN_WORKSPACE_BYTES,     /* workspace of the whole call */
+  SMX_PLAN_WIDE_PAIRS,          /* tiled path on the 256-token tiles: pairs of work ranges the grids
+                                   are sized for; 0: the 128-token tiles, or not tiled */
   SMX_PLAN_FIELDS
 };
 int smx_moe_plan_info(int64_t T, int64_t H, int64_t I, int64_t E, int64_t top_k,

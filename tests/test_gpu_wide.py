@@ -9,11 +9,13 @@ import pytest
 import torch
 
 from oracle import moe_ref as ref
+from ae_amd import _lib
 from ae_amd.layers import fused_moe_shared_forward, stack_fused_moe, tiled_min_tokens
 from tests.helpers import TOL, TORCH_TO_ORACLE, f32_of, make_pool, max_rel_err, to_oracle
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
+DCODE = {torch.float16: _lib.SMX_F16, torch.bfloat16: _lib.SMX_BF16}
 
 
 def _stack(counts, H, I, dtype, seed, unmapped=()):
@@ -29,6 +31,7 @@ def _stack(counts, H, I, dtype, seed, unmapped=()):
         slots[e] = -1
     logits = torch.zeros((T, E), dtype=dtype, device=DEV)
     with tiled_min_tokens(0):
+        assert _lib.plan_info(T, H, I, E, 1, DCODE[dtype])["wide_pairs"] > 0
         y = stack_fused_moe(x.clone(), pool, slots, logits, w, ids, False, inplace=False)
     with tiled_min_tokens(1 << 62):
         ys = stack_fused_moe(x.clone(), pool, slots, logits, w, ids, False, inplace=False)
@@ -69,6 +72,7 @@ def test_wide_shared_expert(dtype, T, Is):
     page = (torch.randn((3 * Is * H,), generator=g, device=DEV) * 0.02).to(dtype)
     pool, slots = make_pool(E, H, I, dtype, num_slots=E + 2, seed=E + 1)
     with tiled_min_tokens(0):
+        assert _lib.plan_info(T, H, I, E, k, DCODE[dtype], Is)["wide_pairs"] > 0
         y = fused_moe_shared_forward(x.clone(), logits, pool, slots, k, True, page, sgate, 1.0, inplace=False)
     torch.cuda.synchronize()
     y_ref, _, _ = ref.fused_moe_shared_forward(

@@ -11,6 +11,7 @@ import numpy as np
 import pytest
 import torch
 
+from ae_amd import _lib
 from ae_amd.layers import stack_fused_moe, tiled_min_tokens
 
 pytestmark = pytest.mark.gpu
@@ -27,7 +28,10 @@ def _layer(x, w1, w3, w2, wide, w=None):
     w = torch.ones((T, 1), device=DEV) if w is None else w
     slots = torch.zeros((1,), dtype=torch.int64, device=DEV)
     logits = torch.zeros((T, 1), dtype=x.dtype, device=DEV)
+    code = _lib.SMX_BF16 if x.dtype == torch.bfloat16 else _lib.SMX_F16
     with tiled_min_tokens(0 if wide else 1 << 62):
+        plan = _lib.plan_info(T, H, I, 1, 1, code)
+        assert (plan["wide_pairs"] > 0, plan["splits"]) == (wide, 1)
         y = stack_fused_moe(x.clone(), pool, slots, logits, w, ids, False, inplace=False)
     torch.cuda.synchronize()
     return y

@@ -12,7 +12,11 @@ It restates, from the device code:
   - tile_down_kernel: reads act rows off + min(q, m-1) over its split's K slice, writes
     part[split][f][owned 16-row tiles] for q < m;
   - combine: reads part[split][t*k+j][:] for every split and every contributing assignment
-    (and the shared expert's part_s[split][t][:]).
+    (and the shared expert's part_s[split][t][:]);
+  - for the wide tiles (wide.hip, the plan's wide_pairs > 0) the same with items of up to 256
+    tokens: wide_item's search for a pair of ranges among the records, wide_range_group, and the
+    token tiles that the waves run for the item's token count. With one K split the routed
+    partials are finished terms in the same rows (one "split").
 Grid sizes, span, splits and split steps come from the library's own host plan
 (smx_moe_plan_info), so the model checks the plan the library launches.
 """
@@ -26,6 +30,9 @@ GATE_COLS = 128         # intermediate columns per gate/up workgroup (kTileGateC
 DOWN_ROWS = 256         # W2 rows per down workgroup (kTileDownRows)
 WAVES = 4
 STEP_BYTES = 64         # unit of split_steps
+WIDE_TOK = 256          # tokens of a wide item (kWideTok)
+WIDE_BLOCK = 4          # token ranges of an expert run side by side (kXBlock)
+WAVE = 64
 
 
 def range_group(local: int, per_item: int, nr: int):
@@ -39,6 +46,23 @@ def range_group(local: int, per_item: int, nr: int):
     inn = local - full
     r = inn // rem
     return r, per_item // 8 * 8 + (inn - r * rem)
+
+
+def wide_range_group(local: int, per_item: int, nr: int):
+    """wide.hip wide_range_group: range_group over blocks of at most WIDE_BLOCK ranges."""
+    nb = -(-nr // WIDE_BLOCK)
+    size = -(-nr // nb)
+    blk = local // (size * per_item)
+    r, g = range_group(local - blk * size * per_item, per_item, min(size, nr - blk * size))
+    return r + blk * size, g
+
+
+def wide_tokens(m: int):
+    """Tokens of a wide item of m that its waves multiply: two groups of waves, each running 16-token
+    tiles group + 2 j for j below twice the item's 64-token quarters."""
+    quarters = -(-m // (WIDE_TOK // 4))
+    assert 1 <= quarters <= 4, m
+    return sorted((wt + 2 * j) * 16 + c for wt in range(2) for j in range(2 * quarters) for c in range(16))
 
 
 def routing_records(ids: np.ndarray, routable: np.ndarray, E: int, span: int):
@@ -79,6 +103,34 @@ def _routed_item(rb: int, per_item: int, recs, span: int):
     return off, m, g
 
 
+def _wide_routed_item(rb: int, per_item: int, recs):
+    """wide_item's routed branch: the (rb / per_item)-th record that begins a pair, found by
+    counting such records 64 at a time (None: past the pairs)."""
+    want = rb // per_item
+    seen, j = 0, -1
+    for base in range(0, len(recs), WAVE):
+        hits = [q for q in range(base, min(base + WAVE, len(recs))) if (q - recs[q]["j0"]) % 2 == 0]
+        if want < seen + len(hits):
+            j = hits[want - seen]
+            break
+        seen += len(hits)
+    if j < 0:
+        return None
+    rr = recs[j]
+    np_ = (rr["nr"] + 1) // 2
+    local = rb - (want - (j - rr["j0"]) // 2) * per_item
+    assert 0 <= local < np_ * per_item, (rb, rr)
+    r, g = wide_range_group(local, per_item, np_)
+    m = min(WIDE_TOK, rr["cnt"] - r * WIDE_TOK)
+    assert m >= 1, (rb, rr, r)
+    return rr["off"] + r * WIDE_TOK, m, g
+
+
+def _wide_shared_item(b: int, per_item: int, tok_groups: int, T: int):
+    r, g = wide_range_group(b, per_item, tok_groups)
+    return r * WIDE_TOK, min(WIDE_TOK, T - r * WIDE_TOK), g
+
+
 def _shared_item(b: int, per_item: int, tok_groups: int, T: int, span: int):
     nr = tok_groups if tok_groups > 1 else 1
     if nr > 1:
@@ -107,13 +159,36 @@ def check_tiled_coverage(T: int, H: int, I: int, k: int, eb: int, ids: np.ndarra
     nranges = len(recs)
     assert nranges <= plan["max_ranges"], f"{nranges} ranges, grid sized for {plan['max_ranges']}"
 
+    wide = plan["wide_pairs"] > 0
+    items_max = plan["wide_pairs"] if wide else plan["max_ranges"]
+    if wide:
+        pairs = sum(1 for q, rr in enumerate(recs) if (q - rr["j0"]) % 2 == 0)
+        assert pairs <= items_max, f"{pairs} pairs, grid sized for {items_max}"
+
+    def shared_item(b: int, per_item: int):
+        if wide:
+            off, m, g = _wide_shared_item(b, per_item, plan["shared_tok_groups"], T)
+        else:
+            off, m, g = _shared_item(b, per_item, plan["shared_tok_groups"], T, span)
+        return _run_tokens(off, m, g)
+
+    def routed_item(rb: int, per_item: int):
+        it = _wide_routed_item(rb, per_item, recs) if wide else _routed_item(rb, per_item, recs, span)
+        return None if it is None else _run_tokens(*it)
+
+    def _run_tokens(off: int, m: int, g: int):
+        if wide:
+            run = wide_tokens(m)
+            assert run[:m] == list(range(m)), "a token of the item runs in no tile, or in two"
+        return off, m, g
+
     s_blocks_gu = plan["shared_gateup_blocks"]
     s_blocks_dn = plan["shared_down_blocks"]
     groups_r = -(-I // GATE_COLS)
     groups_s = -(-Is // GATE_COLS) if Is else 0
     rgroups = -(-H // DOWN_ROWS)
-    assert plan["tile_gateup_grid"] == s_blocks_gu + plan["max_ranges"] * groups_r
-    assert plan["tile_down_grid"] == s_blocks_dn + plan["max_ranges"] * rgroups * plan["splits"]
+    assert plan["tile_gateup_grid"] == s_blocks_gu + items_max * groups_r
+    assert plan["tile_down_grid"] == s_blocks_dn + items_max * rgroups * plan["splits"]
 
     # gate/up: act [N, I/16] and act_s [T, Is/16] written
     act = np.zeros((N, I // ROW_TILE), dtype=np.int32)
@@ -121,12 +196,12 @@ def check_tiled_coverage(T: int, H: int, I: int, k: int, eb: int, ids: np.ndarra
     items = 0
     for b in range(plan["tile_gateup_grid"]):
         if b < s_blocks_gu:
-            off, m, g = _shared_item(b, groups_s, plan["shared_tok_groups"], T, span)
+            off, m, g = shared_item(b, groups_s)
             tiles = [t for w in range(WAVES) for t in
                      _owned_tiles(g * GATE_COLS // ROW_TILE + 2 * w, 2, Is // ROW_TILE - 1)]
             act_s[off:off + m, tiles] += 1
         else:
-            it = _routed_item(b - s_blocks_gu, groups_r, recs, span)
+            it = routed_item(b - s_blocks_gu, groups_r)
             if it is None:
                 continue
             off, m, g = it
@@ -154,7 +229,7 @@ def check_tiled_coverage(T: int, H: int, I: int, k: int, eb: int, ids: np.ndarra
     part_s = np.zeros((max(s_splits, 1), T, H // ROW_TILE), dtype=np.int32)
     for b in range(plan["tile_down_grid"]):
         if b < s_blocks_dn:
-            off, m, g = _shared_item(b, rgroups * s_splits, plan["shared_tok_groups"], T, span)
+            off, m, g = shared_item(b, rgroups * s_splits)
             sp, rg = divmod(g, rgroups)
             c0, c1 = k_cols(sp, plan["shared_split_steps"], Is)
             assert (act_s[off:off + m, c0:c1] == 1).all(), "shared down reads an unwritten act row"
@@ -162,13 +237,13 @@ def check_tiled_coverage(T: int, H: int, I: int, k: int, eb: int, ids: np.ndarra
             for q in range(m):
                 part_s[sp, off + q, tiles] += 1
         else:
-            it = _routed_item(b - s_blocks_dn, rgroups * splits, recs, span)
+            it = routed_item(b - s_blocks_dn, rgroups * splits)
             if it is None:
                 continue
             off, m, g = it
             sp, rg = divmod(g, rgroups)
             c0, c1 = k_cols(sp, plan["split_steps"], I)
-            # token rows off + min(q, m - 1), q < 128: exactly rows [off, off + m)
+            # token rows off + min(q, m - 1): exactly rows [off, off + m)
             assert (act[off:off + m, c0:c1] == 1).all(), "down reads an unwritten act row"
             tiles = [t for w in range(WAVES) for t in _owned_tiles(rg * DOWN_ROWS // ROW_TILE + 4 * w, 4, H // ROW_TILE - 1)]
             for q in range(m):
