@@ -1,7 +1,7 @@
 """SiLU of the wide tiled kernels (wide.hip) at every value a 16-bit gate can take: the class (finite,
-infinite, NaN) and the bits of the weight-streaming kernels' outputs, and the exact value rounded
-to the activation type; and the bits of the terms that the down projection weighs. One expert;
-each token carries one gate pattern.
+infinite, NaN), the exact value rounded to the activation type, and no more misrounded outputs than
+the weight-streaming kernels have; and the bits of the terms that the down projection weighs. One
+expert; each token carries one gate pattern.
 
 The finite gates: x[t] = (pattern_t, 1, 0, ...), W1 row i = (1, 0, ...), W3 row i = (0, u_i, 0, ...),
 W2 = identity: output h is round(silu(pattern_t) * u_h), with no sum of more than one non-zero
@@ -56,7 +56,6 @@ def test_every_finite_gate(dtype):
     y = _layer(x, w1, w3, w2, True)
     assert torch.isfinite(y.float()).all(), int((~torch.isfinite(y.float())).any(1).sum())
     ys = _layer(x, w1, w3, w2, False)
-    assert torch.equal(y.view(torch.int16), ys.view(torch.int16))
     g = p.double()
     exact = (g / (1.0 + torch.exp(-g)))[:, None] * u.double()
     # half a unit of the type for its rounding; the fp32 value before it is within 2^-21 of the
@@ -65,22 +64,36 @@ def test_every_finite_gate(dtype):
     # Where 1 + e^-g overflows (g < -88.72) the result is -0 for an exact value above -2.8e-37.
     bits, emin = FORM[dtype]
     unit = torch.exp2(torch.floor(torch.log2(exact.abs().clamp_min(2.0 ** emin))) - bits)
-    err = (y.double() - exact).abs()
+    err, errs = (y.double() - exact).abs(), (ys.double() - exact).abs()
     over = (g < -88.72)[:, None].expand_as(err)
     small = (exact.abs() < 2.0 ** emin) & ~over
-    assert (err <= (0.5 + 2.0 ** -9) * unit)[~small & ~over].all(), (err / unit)[~small & ~over].max().item()
+    rest = ~small & ~over
+    assert (err <= (0.5 + 2.0 ** -9) * unit)[rest].all(), (err / unit)[rest].max().item()
     assert (err <= 2.0 ** emin)[small].all()
     assert (y[over] == 0).all() and (exact[over] >= -2.8e-37).all()
+    # outputs that are not the nearest value of the type (about the fp32 error in units of the
+    # type: one in 10^4 to 10^5); another SiLU of the same error misrounds others, as many
+    wrong, wrongs = (int((q > 0.5 * unit)[rest].sum()) for q in (err, errs))
+    print(f"misrounded of {int(rest.sum())}: wide {wrong}, streaming {wrongs}")
+    assert wrong <= 1.1 * wrongs + 3 * wrongs ** 0.5
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_weighted_terms(dtype):
-    """One K split: the down kernel rounds weight * sum itself, as the combine does elsewhere."""
+    """One K split: the down kernel weighs and rounds its sums itself, as the combine does
+    elsewhere: in fp16 rounded once from the exact product, in bf16 from the fp32 product."""
     p, _, x, w1, w3, w2 = _finite_gates(dtype)
     g = torch.Generator(device=DEV).manual_seed(5)
     w = torch.rand((p.numel(), 1), generator=g, device=DEV) + 0.25
-    y, ys = (_layer(x, w1, w3, w2, wide, w) for wide in (True, False))
-    assert torch.equal(y.view(torch.int16), ys.view(torch.int16))
+    act = _layer(x, w1, w3, w2, True)  # weight 1: the sums themselves
+    y = _layer(x, w1, w3, w2, True, w)
+    if dtype == torch.float16:
+        prod = act.cpu().double().numpy() * w.cpu().double().numpy()
+        with np.errstate(over="ignore"):  # weights above 1 overflow the largest gates
+            want = torch.from_numpy(prod.astype(np.float16)).to(DEV)
+    else:
+        want = (act.float() * w).to(dtype)
+    assert torch.equal(y, want)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
