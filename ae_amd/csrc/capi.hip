@@ -236,14 +236,22 @@ int64_t divisor_at_most(int64_t n, int64_t want) {
 // fills the chip (the routing decides the last round). Measured, down + combine in us per call:
 // Mixtral with 1 / 2 / 4 splits, 8192 tokens 1765 / 1823 / 1977, 4096: 974 / 974 / 1082, 2048: 671 /
 // 577 / 588, 1025: 388 / 373 / 359 (before this rule: 4 splits at 2048, 1590 -> 1450 us per call).
+// Walks of at most kWideUnsplitSteps steps stay whole: their steps read a few MB and take ~0.3 us,
+// not kWideStepUs, so that a split saves less than its partials cost. Us per call, 8 experts, top-2,
+// split -> whole (128-token tiles): hidden = ffn = 256 (4 steps), 512 tokens 40.9 -> 39.1 (39.9),
+// 2048: 49.6 -> 45.6 (48.4); hidden 512, ffn 384 (6 steps), 600 tokens fp16 50.5 -> 47.5 (43.0). At
+// 8 steps it depends on the load: hidden = ffn = 512, 512 tokens 50.5 -> 48.3, 2048: 56.6 -> 57.9;
+// hidden 1024, ffn 512, 600 tokens 59.6 -> 61.0.
 constexpr double kWideStepUs = 1.5;         // one 128-byte K step of a 256 x 256 tile
 constexpr double kWideFixedSteps = 5.0;     // start and end of a workgroup, in steps
 constexpr double kWidePartBytesPerUs = 4.5e6;
 constexpr int64_t kWideMaxSplits = 16;
+constexpr int64_t kWideUnsplitSteps = 6;
 int64_t wide_splits(int64_t N, double active, int64_t T, int64_t H, int64_t nsteps, int64_t ssteps, int64_t most) {
   const int64_t rgroups = (H + kTileDownRows - 1) / kTileDownRows;
   const double tiles = static_cast<double>(N) / kWideTok + 0.5 * active;
   const int64_t sgroups = (T + kWideTok - 1) / kWideTok;
+  if (nsteps <= kWideUnsplitSteps) most = 1;
   int64_t best = 1;
   double best_us = 0.0;
   for (int64_t s = 1; s <= most && s <= nsteps / 2; ++s) {

@@ -18,7 +18,7 @@ DEV = "cuda"
 DCODE = {torch.float16: _lib.SMX_F16, torch.bfloat16: _lib.SMX_BF16}
 
 
-def _stack(counts, H, I, dtype, seed, unmapped=()):
+def _stack(counts, H, I, dtype, seed, unmapped=(), splits=1):
     """Every token picks one expert (k = 1): expert e gets counts[e] tokens, in a shuffled order."""
     E, T = len(counts), sum(counts)
     g = torch.Generator(device=DEV).manual_seed(seed)
@@ -31,7 +31,8 @@ def _stack(counts, H, I, dtype, seed, unmapped=()):
         slots[e] = -1
     logits = torch.zeros((T, E), dtype=dtype, device=DEV)
     with tiled_min_tokens(0):
-        assert _lib.plan_info(T, H, I, E, 1, DCODE[dtype])["wide_pairs"] > 0
+        plan = _lib.plan_info(T, H, I, E, 1, DCODE[dtype])
+        assert plan["wide_pairs"] > 0 and plan["splits"] == splits
         y = stack_fused_moe(x.clone(), pool, slots, logits, w, ids, False, inplace=False)
     with tiled_min_tokens(1 << 62):
         ys = stack_fused_moe(x.clone(), pool, slots, logits, w, ids, False, inplace=False)
@@ -55,6 +56,17 @@ def _stack(counts, H, I, dtype, seed, unmapped=()):
 ])
 def test_wide_token_counts(dtype, counts, H, I):
     _stack(counts, H, I, dtype, seed=sum(counts) + H)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("counts,H,I,splits", [
+    ([2049, 0, 1], 128, 640, 5),
+    ([63, 64, 65, 320], 256, 1024, 8),
+    ([127, 128, 129, 191, 192, 193], 384, 1152, 9),
+])
+def test_wide_partials(dtype, counts, H, I, splits):
+    """Walks of more than 6 steps: K splits, whose fp32 partials the combine adds."""
+    _stack(counts, H, I, dtype, seed=sum(counts) + I, splits=splits)
 
 
 def test_wide_dropped_assignments():

@@ -155,7 +155,7 @@ WIDE_COUNTS = [[1, 511], [63, 64, 65, 320], [127, 128, 129, 191, 192, 193], [255
 
 
 @pytest.mark.parametrize("counts", WIDE_COUNTS)
-@pytest.mark.parametrize("H,I,Is", [(128, 128, 0), (384, 256, 0), (256, 128, 384)])
+@pytest.mark.parametrize("H,I,Is", [(128, 128, 0), (384, 640, 0), (256, 128, 384)])
 def test_wide_items(counts, H, I, Is):
     E = len(counts)
     ids = np.repeat(np.arange(E), counts)
@@ -170,7 +170,7 @@ def test_wide_items(counts, H, I, Is):
 
 @pytest.mark.parametrize("splits_one", [True, False])
 def test_wide_dropped_assignments(splits_one):
-    T, H, I, E, k = 900, 256, 128 if splits_one else 512, 8, 2
+    T, H, I, E, k = 900, 256, 128 if splits_one else 1024, 8, 2
     ids = _topk(np.random.default_rng(9).standard_normal((T, E)), k)
     routable = ~np.isin(ids, [2, 5])
     with tiled_threshold(0):
