@@ -36,10 +36,12 @@ constexpr int64_t kDownFillBlocks = 512;  // one residency: two down workgroups 
 // (measured crossover: Mixtral 64 tokens per expert 613 vs 637 us, 32: 590 vs 502 us;
 // Qwen1.5-MoE 68: 378 vs 466 us, 34: 456 vs 293 us).
 constexpr int64_t kTileTargetDownBlocks = 512;
-// From this many expected tokens per active expert the down projection aims for 4x the
-// workgroups: with ~2 rounds of workgroups the last round ran mostly empty (Mixtral 4096 tokens:
-// 1072 workgroups on 512 slots; 2 K splits: down 1164 -> 1035 us, the combine's extra split 33 ->
-// 56 us). Below it the extra splits cost more in the combine than they save.
+// From this many expected tokens per active expert the down projection of the 128-token tiles aims
+// for 4x the workgroups (fp32; 16-bit batches of that size run on the wide tiles, for which this
+// split count is only a bound on the workspace): with ~2 rounds of workgroups the last round ran
+// mostly empty. fp32, 1 / 2 / 4 K splits in us per call: Mixtral 2048 tokens 13889 / 12434 / 11767 (down
+// 6308 / 4747 / 4040), 4096 tokens 23181 / 21755 / 21381; hidden = ffn = 2048, 2048 tokens 1329 / 1314 /
+// 1248. Below it the extra splits cost more in the combine than they save.
 constexpr int64_t kTileLargeTokens = 512;
 // Batches from this many tokens combine with one thread per 8 outputs (combine_rows_kernel);
 // smaller ones with one workgroup per (token, 256 outputs), one wave per assignment. Measured
@@ -48,11 +50,25 @@ constexpr int64_t kTileLargeTokens = 512;
 constexpr int64_t kCombineRowsMinTokens = 128;
 constexpr int64_t kTileMinTokensDefault = 64;
 // Tiled batches of 16-bit types from this many expected tokens per active expert run on the wide
-// tiles (wide.hip, 256 tokens x 256 weight rows) instead of the 128-token tiles: below it their
-// second half is mostly padding and the weights bound the call. Measured per call, 128-token ->
-// wide tiles, at the expected tokens per expert: Mixtral 100: 682 -> 708 us, DeepSeek-V2-Lite 103:
-// 331 -> 369, Qwen1.5-MoE 133: 497 -> 445, Mixtral 175: 822 -> 815, DeepSeek-V2-Lite 192: 490 ->
-// 457, Mixtral 256: 1057 -> 950, 2048: 5705 -> 4850.
+// tiles (wide.hip, 256 tokens x 256 weight rows) instead of the 128-token tiles: from there an
+// expert of the expected size needs two ranges of 128, and one wide item. Below it the item's second
+// half is padding and the weights bound the call. Us per call, 128-token -> wide tiles, at the
+// expected tokens per expert (bf16; a skewed load is Zipf, s = 1.2):
+//   below: Mixtral 100 skewed: 682 -> 708, 120: 667 -> 689, 120 skewed: 675 -> 715, DeepSeek-V2-Lite 103:
+//     331 -> 369;
+//   at 128: Mixtral 727 -> 689, skewed 671 -> 718 (fp16 677 -> 697), Mixtral-8x22B skewed 1212 -> 1180,
+//     DBRX 1607 -> 1436, Qwen1.5-MoE 475 -> 413, DeepSeek-V2-Lite 386 -> 370;
+//   above: Mixtral skewed 129: 725 -> 702, 136: 757 -> 742 (fp16 740 -> 733), 144: 812 -> 785 (fp16 775 ->
+//     751), 160: 818 -> 800 (fp16 822 -> 805), 176: 822 -> 823, 192: 852 -> 830, 256: 1057 -> 950, 2048:
+//     5705 -> 4800; Mixtral 132: 773 -> 706, 150: 837 -> 729; DeepSeek-V2-Lite 141: 440 -> 382, 192: 490 ->
+//     457; Qwen1.5-MoE 140: 521 -> 449.
+// The plan does not know the load. Where the wide grid is about one round of the chip or less, a
+// skewed load costs it up to 12 % (fp16 17 %) between 128 and 230 tokens per expert (its busiest
+// expert's full items end last, or begin a second round), and a balanced one gains more: 8 experts
+// of hidden 4096, ffn 3584, 150 tokens per expert 246 -> 194, skewed 234 -> 265; ffn 1792, 128: 177 ->
+// 146, 150: 149 -> 149, skewed 149 -> 160, 192: 153 -> 166, skewed 153 -> 167; hidden 1024, ffn 512, 128:
+// 58.0 -> 47.8, skewed 57.8 -> 58.3 (fp16, 150: 51.9 -> 49.0, skewed 52.3 -> 59.9). No cut by the grid's
+// size separates the two.
 constexpr double kWideMinTokens = 128.0;
 int64_t g_tile_min_tokens = kTileMinTokensDefault;
 // Batches of at most this many tokens run the down projection and the combine as one kernel
@@ -327,8 +343,13 @@ Plan make_plan(int64_t T, int64_t H, int64_t I, int64_t E, int64_t k, int dtype,
     s = divisor_at_least(nsteps / 2, want);
     if (s > 4 * want) s = divisor_at_most(nsteps / 2, want);
     if (wide) {
-      // a batch whose partials of the 128-token tiles' split count fit the scratch of
-      // smx_fused_moe_forward_noalloc takes at most that many splits: its workspace does not grow
+      // A batch whose partials of the 128-token tiles' split count fit the scratch of
+      // smx_fused_moe_forward_noalloc takes at most that many splits, so that no call outgrows the
+      // scratch by its tiles (at most as many splits of either expert, the rest of the workspace
+      // the same). This holds for every entry point: all give the same bits for the same call.
+      // Past it the workspace may be up to 1.6 times the 128-token tiles' (Mixtral 600 tokens 70 ->
+      // 107 MB, 1025: 120 -> 184, Mixtral-8x22B 600: 93 -> 150, DBRX 600: 105 -> 161), for 20 us of 800
+      // in Mixtral's calls, or half of it (Mixtral 2048 tokens 368 -> 240).
       const size_t part = sizeof(float) * static_cast<size_t>(s) * static_cast<size_t>(p.N * H);
       s = wide_splits(p.N, active, T, H, nsteps, Is * eb / 128,
                       part <= SMX_NOALLOC_SCRATCH_BYTES ? s : kWideMaxSplits);
