@@ -383,6 +383,19 @@ __device__ __forceinline__ u32x4 join_tiles(const u32x2& a, const u32x2& b) {
 // The lane's first column of a joined pair of tiles.
 __device__ __forceinline__ int join_col(int lane) { return ((lane >> 4) & 1) * kRowTile + (lane >> 5) * 8; }
 
+// A copy of an accumulator, made here: without the assembly the compiler moved all of a wave's 256
+// accumulator registers to vector registers ahead of the branches of the epilogue, and spilled.
+__device__ __forceinline__ f32x4 acc_read(const f32x4& acc) {
+  f32x4 v;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    float x;
+    asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(x) : "a"(acc[e]));
+    v[e] = x;
+  }
+  return v;
+}
+
 struct WideStages {
   u32x4 *a0, *b0, *a1, *b1;
 };
@@ -453,7 +466,7 @@ __device__ __forceinline__ void wide_down_item(const ExpertArgs& a, const WorkIt
         u32x2 v[2];
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
-          const f32x4 d = acc[i + p][j];
+          const f32x4 d = acc_read(acc[i + p][j]);
           v[p] = u32x2{mul2<DT>(f32x2{d[0], d[1]}, wf), mul2<DT>(f32x2{d[2], d[3]}, wf)};
         }
         const u32x4 o = join_tiles(v[0], v[1]);

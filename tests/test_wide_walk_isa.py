@@ -8,9 +8,10 @@ of the K walk in the compiled code (two steps per iteration, one loop per token-
   - at least two instructions before the first MFMA, and `s_nop 15` after the last one, before
     anything can read an accumulator;
   - each of the two barriers directly follows a wait for every DMA and LDS read of the wave, and
-    each is followed by one step's DMA (8 weight and 2, 4, 6 or 8 token instructions).
+    each is followed by one step's DMA (8 weight and 2, 4, 6 or 8 token instructions);
 
-Runs on the CPU: hipcc cross-compiles; no GPU is used."""
+and that no kernel spills registers to scratch memory. Runs on the CPU: hipcc cross-compiles; no GPU
+is used."""
 import os
 import re
 import shutil
@@ -33,12 +34,12 @@ def wide_loops(tmp_path_factory):
            os.path.join(libbuild.CSRC, "wide.hip"), "-o", str(out)]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     assert proc.returncode == 0, proc.stderr
-    loops, kernel, label, body = {}, None, None, []
+    loops, spills, kernel, label, body = {}, {}, None, None, []
     for line in out.read_text().split("\n"):
         m = KERNEL_RE.match(line)
         if m:
             kernel, label, body = m.group(1), None, []
-            loops[kernel] = []
+            loops[kernel], spills[kernel] = [], []
         elif line.startswith(".Lfunc_end"):
             kernel = None
         elif kernel and re.match(r"^\.LBB\w+:", line):
@@ -47,12 +48,20 @@ def wide_loops(tmp_path_factory):
             t = line.split(";")[0].strip()
             if t and not t.startswith("."):
                 body.append(t)
+                if t.startswith("scratch_"):
+                    spills[kernel].append(t)
                 if t.startswith("s_cbranch") and t.split()[-1] == label and any("v_mfma" in b for b in body):
                     loops[kernel].append(body)
-    return loops
+    return loops, spills
+
+
+def test_no_spills(wide_loops):
+    assert len(wide_loops[1]) == 6
+    assert {k: v for k, v in wide_loops[1].items() if v} == {}
 
 
 def test_walk_loops(wide_loops):
+    wide_loops = wide_loops[0]
     assert len(wide_loops) == 6, sorted(wide_loops)  # gate/up, down of partials and of terms; fp16 and bf16
     for name, loops in wide_loops.items():
         tiles = sorted(sum("v_mfma" in t for t in b) // 32 for b in loops)
