@@ -10,8 +10,10 @@ import torch
 
 from oracle import moe_ref as ref
 from ae_amd import _lib
-from ae_amd.layers import fused_moe_shared_forward, stack_fused_moe, tiled_min_tokens
-from tests.helpers import TOL, TORCH_TO_ORACLE, f32_of, make_pool, max_rel_err, to_oracle
+from ae_amd.layers import (fused_moe_shared_forward, stack_fused_moe, stack_fused_moe_shared,
+                           tiled_min_tokens)
+from tests.helpers import (TOL, TORCH_TO_ORACLE, f32_of, make_pool, max_rel_err, nan_buffers,
+                           to_oracle)
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -69,8 +71,45 @@ def test_wide_partials(dtype, counts, H, I, splits):
     _stack(counts, H, I, dtype, seed=sum(counts) + I, splits=splits)
 
 
-def test_wide_dropped_assignments():
-    _stack([300, 150, 257, 129], 256, 256, torch.bfloat16, seed=7, unmapped=(1,))
+@pytest.mark.parametrize("I,splits", [(256, 1), (1024, 8)])
+def test_wide_dropped_assignments(I, splits):
+    _stack([300, 150, 257, 129], 256, I, torch.bfloat16, seed=7, unmapped=(1,), splits=splits)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("I,splits", [(128, 1), (1024, 4)])
+@pytest.mark.parametrize("Is", [0, 384])
+def test_wide_dropped_picks_of_a_token(dtype, I, splits, Is):
+    """Tokens with some and with all of their three picks dropped (an unmapped expert, ids outside the
+    experts), on an output of NaN and a workspace of 0xFF bytes: a row of terms or partials that the
+    down kernel did not write is not added."""
+    T, H, E, k = 700, 256, 6, 3
+    r = np.random.default_rng(I + Is)
+    ids = np.argsort(r.random((T, E)), axis=1)[:, :k].astype(np.int32)
+    ids[r.random((T, k)) < 0.1] = -1
+    ids[::7] = [2, -1, E]  # expert 2 is unmapped: nothing is left of these
+    w = (r.random((T, k)) + 0.2).astype(np.float32)
+    g = torch.Generator(device=DEV).manual_seed(T)
+    x = torch.randn((T, H), generator=g, device=DEV).to(dtype)
+    page = (torch.randn((3 * Is * H,), generator=g, device=DEV) * 0.02).to(dtype) if Is else None
+    sgate = torch.randn((T, 1), generator=g, device=DEV).to(dtype) if Is else None
+    pool, slots = make_pool(E, H, I, dtype, num_slots=E + 2, seed=E)
+    slots[2] = -1
+    with tiled_min_tokens(0):
+        plan = _lib.plan_info(T, H, I, E, k, DCODE[dtype], Is)
+        assert plan["wide_pairs"] > 0 and plan["splits"] == splits
+        nbytes = _lib.lib().smx_moe_shared_workspace_size(T, H, I, E, k, Is, DCODE[dtype])
+        out, ws = nan_buffers(x, nbytes)
+        y = stack_fused_moe_shared(x, pool, slots, torch.from_numpy(w).to(DEV), torch.from_numpy(ids).to(DEV),
+                                   page, sgate, 1.0, inplace=False, out=out, workspace=ws)
+    torch.cuda.synchronize()
+    assert torch.isfinite(y.float()).all()
+    y_ref = ref.stack_fused_moe_shared(to_oracle(x), to_oracle(pool), slots.cpu().numpy(), w, ids,
+                                       TORCH_TO_ORACLE[dtype], shared_page=None if page is None else to_oracle(page),
+                                       shared_gate_logits=None if sgate is None else f32_of(sgate))
+    assert max_rel_err(f32_of(y), y_ref) <= TOL[dtype]
+    if not Is:
+        assert (y[::7] == 0).all()
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
