@@ -245,3 +245,55 @@ def test_layer_module_grouped_routing_block(method):
                                        shared_page=to_oracle(blk.shared_ws.data),
                                        routed_scaling_factor=2.5)
     assert max_rel_err(f32_of(y), y_ref) <= TOL[dt]
+
+
+# Past 512 tokens the norm + gate kernel keeps the token's row in dynamic LDS, sized by H. One more
+# token must not change the others' bits, at the largest row and for every form of the gate.
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("H,E", [(128, 0), (2048, 8), (4096, 60), (1024, 256), (16384, 64), (16384, 0)])
+def test_norm_gate_rows_on_both_sides_of_the_lds_rule(dtype, H, E):
+    x = _rand((513, H), dtype, seed=H + E, scale=2.0)
+    r = _rand((513, H), dtype, seed=H + E + 1)
+    w = _rand((H,), dtype, seed=H, scale=0.2) + 1
+    gw = _rand((E, H), dtype, seed=E + 2, scale=0.02) if E else None
+    res = {}
+    for T in (512, 513):
+        xn, rn = x[:T].clone(), r[:T].clone()
+        lg = add_rmsnorm_gate(xn, rn, w, 1e-6, gate_weight=gw)
+        torch.cuda.synchronize()
+        res[T] = (xn, rn) + ((lg,) if E else ())
+    for a, b in zip(res[512], res[513]):
+        assert torch.equal(a, b[:512])
+    xn_ref, res_ref = ref.add_rmsnorm(to_oracle(x[500:]), to_oracle(r[500:]), to_oracle(w), 1e-6, TORCH_TO_ORACLE[dtype])
+    np.testing.assert_array_equal(f32_of(res[513][1][500:]), res_ref)
+    _check_normed(res[513][0][500:], xn_ref, dtype)
+    if E:
+        lg_ref = ref.router_logits(to_oracle(res[513][0][500:]), to_oracle(gw), TORCH_TO_ORACLE[dtype])
+        tol = {torch.bfloat16: 1e-2, torch.float16: 2e-3, torch.float32: 1e-5}[dtype]
+        assert max_rel_err(f32_of(res[513][2][500:]), lg_ref) <= tol
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("E,k", [(8, 2), (16, 4), (30, 3), (60, 4), (200, 8)])
+def test_layer_routing_on_both_sides_of_the_lds_rule(dtype, E, k):
+    """The same for the layer call: residual, logits and the top-k of every lane-group form."""
+    H, I, Is = 256, 128, 128
+    x, r = _rand((513, H), dtype, seed=E), _rand((513, H), dtype, seed=E + 1)
+    nw = _rand((H,), dtype, seed=E + 2, scale=0.1) + 1
+    gw, sgw = _rand((E, H), dtype, seed=E + 3, scale=0.05), _rand((H,), dtype, seed=E + 4, scale=0.05)
+    page = _rand((3 * Is * H,), dtype, seed=E + 5, scale=0.02)
+    pool, slots = make_pool(E, H, I, dtype, num_slots=E, seed=E + 6)
+    res = {}
+    for T in (512, 513):
+        rn = r[:T].clone()
+        _, (lg, w, ids) = moe_layer_forward(x[:T].clone(), rn, nw, 1e-6, gw, pool, slots, k, False, shared_w=page,
+                                            shared_gate_weight=sgw, return_routing=True)
+        torch.cuda.synchronize()
+        res[T] = (rn, lg, w, ids)
+    for a, b in zip(res[512], res[513]):
+        assert torch.equal(a, b[:512])
+
+
+@pytest.mark.parametrize("E,k,Is,gated", [(60, 4, 256, True), (8, 2, 0, False)])
+def test_layer_forward_past_the_lds_rule(E, k, Is, gated):
+    _layer_case(513, 256, 128, E, k, E <= 8, Is=Is, gated=gated, seed=600 + E)
