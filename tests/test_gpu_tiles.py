@@ -9,7 +9,8 @@ import pytest
 import torch
 
 from oracle import moe_ref as ref
-from ae_amd.layers import fused_moe_forward, fused_moe_shared_forward, tiled_min_tokens
+from ae_amd.layers import (fused_moe_forward, fused_moe_shared_forward, stack_fused_moe_shared,
+                           tiled_min_tokens)
 from ae_amd import _lib
 from tests.helpers import (TOL, TORCH_TO_ORACLE, f32_of, make_pool, max_rel_err, nan_buffers,
                            to_oracle, zipf_gate_logits)
@@ -201,3 +202,30 @@ def test_mixtral_max_assignments_sampled(path):
     del pool
     err = max_rel_err(f32_of(y[rows.to(DEV)]), y_ref)
     assert err <= TOL[torch.bfloat16], err
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,I", [(256, 128), (384, 640)])
+def test_tiled_many_ranges_below_the_wide_tiles(dtype, H, I):
+    """16-bit types on the 128-token tiles over several ranges of an expert: a caller's skewed
+    routing whose expected tokens per expert (100) stay below the 256-token tiles."""
+    counts = [700, 300, 257, 129, 128, 65, 1, 20] + [0] * 8
+    E, T = len(counts), sum(counts)
+    ids = np.repeat(np.arange(E, dtype=np.int32), counts)
+    np.random.default_rng(H).shuffle(ids)
+    x, logits = _inputs(T, H, E, dtype, seed=H + I)
+    w = (np.random.default_rng(I).random((T, 1)) + 0.5).astype(np.float32)
+    pool, slots = make_pool(E, H, I, dtype, num_slots=E + 2, seed=I)
+    with tiled_min_tokens(0):
+        code = {torch.bfloat16: _lib.SMX_BF16, torch.float16: _lib.SMX_F16}[dtype]
+        plan = _lib.plan_info(T, H, I, E, 1, code)
+        assert plan["tiled"] == 1 and plan["wide_pairs"] == 0
+        out, ws = _poisoned(x, logits, pool, 1)
+        y = stack_fused_moe_shared(x, pool, slots, torch.from_numpy(w).to(DEV),
+                                   torch.from_numpy(ids[:, None].copy()).to(DEV), None, None, 1.0,
+                                   inplace=False, out=out, workspace=ws)
+    torch.cuda.synchronize()
+    assert torch.isfinite(y.float()).all()
+    y_ref = ref.stack_fused_moe(to_oracle(x), to_oracle(pool), slots.cpu().numpy(), w, ids[:, None],
+                                TORCH_TO_ORACLE[dtype])
+    assert max_rel_err(f32_of(y), y_ref) <= TOL[dtype]
