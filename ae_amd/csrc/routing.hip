@@ -918,11 +918,18 @@ hipError_t launch_route(const void* logits, int ldt, int T, int E, int k, int re
 
 template <int DT, int G, int PL, int RB>
 static void norm_gate_launch(const NormGateArgs& a, hipStream_t s) {
-  // LDS for the token's row only, so that a CU holds as many workgroups as that leaves room for --
-  // two with the largest row's fixed 64 KB, too few to cover the gate rows' L2 latency
-  // (DeepSeek-V2-Lite layer of 2047 tokens 483.6 -> 475.8 us). A batch that two workgroups per CU
-  // hold keeps the fixed row (32 tokens 187.1 us against 188.2).
-  if (a.T > 2 * kNormCUs)
+  // LDS for the token's row only (kDyn) where the workgroups that then fit a CU's LDS, against two with
+  // the largest row's fixed 64 KB, finish the batch in fewer rounds. In equal rounds the fixed form is
+  // faster: the compiler knows its two workgroups per CU and keeps more of the gate rows in
+  // registers. Norm + gate alone, us, fixed / dynamic, bf16 unless said: hidden 2048, 64 experts, 512 tokens
+  // 11.8 / 11.7, 640: 14.8 / 12.0, 2048: 32.4 / 28.1; hidden 4096, 8 experts, 640: 13.7 / 11.8, 2048: 26.7 /
+  // 21.9 (fp32 36.3 / 29.0); hidden 5120, 160 experts, 512: 35.9 / 40.7, 640: 59.9 / 44.9, 2048: 133 / 125;
+  // hidden 8192, 128 experts, 640: 74.2 / 56.6, 1024: 86.2 / 90.0 (fp32 151 / 153), 2048: 175 / 170 (304 /
+  // 310); hidden 12288 (three per CU), 64 experts, 640: 69.5 / 50.6, 1024 (two rounds of either): 82.2 /
+  // 96.6, 1280: 118 / 105, 4096: 349 / 316; hidden 16384 (two), 640: 88.0 / 101.5, 2048: 219 / 241.
+  const int fit = kNormCuLds / (static_cast<int>(sizeof(float)) * a.H + kNormFixedLds);
+  auto rounds = [&](int per_cu) { return (a.T + kNormCUs * per_cu - 1) / (kNormCUs * per_cu); };
+  if (fit > 2 && rounds(fit) < rounds(2))
     norm_gate_kernel<DT, G, PL, RB, true><<<a.T, kNormThreads, sizeof(float) * a.H, s>>>(a);
   else
     norm_gate_kernel<DT, G, PL, RB, false><<<a.T, kNormThreads, 0, s>>>(a);

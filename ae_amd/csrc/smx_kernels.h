@@ -231,6 +231,8 @@ hipError_t launch_layer1(int dtype, const ExpertArgs& a, int max_ranges, int rou
 constexpr int kNormThreads = 256;
 constexpr int kNormWaves = kNormThreads / kWave;
 constexpr int kNormCUs = 256;     // compute units of the chip
+constexpr int kNormCuLds = 160 * 1024;    // LDS of a compute unit
+constexpr int kNormFixedLds = 2560;       // past the row: logits, partial sums, allocation granule
 constexpr int kNormMaxH = 16384;  // one token's fp32 row is staged in LDS
 
 struct NormGateArgs {
