@@ -60,7 +60,7 @@ constexpr int64_t kTileMinTokensDefault = 64;
 //     DBRX 1607 -> 1436, Qwen1.5-MoE 475 -> 413, DeepSeek-V2-Lite 386 -> 370;
 //   above: Mixtral skewed 129: 725 -> 702, 136: 757 -> 742 (fp16 740 -> 733), 144: 812 -> 785 (fp16 775 ->
 //     751), 160: 818 -> 800 (fp16 822 -> 805), 176: 822 -> 823, 192: 852 -> 830, 256: 1057 -> 950, 2048:
-//     5705 -> 4800; Mixtral 132: 773 -> 706, 150: 837 -> 729; DeepSeek-V2-Lite 141: 440 -> 382, 192: 490 ->
+//     5705 -> 4770; Mixtral 132: 773 -> 706, 150: 837 -> 729; DeepSeek-V2-Lite 141: 440 -> 382, 192: 490 ->
 //     457; Qwen1.5-MoE 140: 521 -> 449.
 // The plan does not know the load. Where the wide grid is about one round of the chip or less, a
 // skewed load costs it up to 12 % (fp16 17 %) between 128 and 230 tokens per expert (its busiest

@@ -3,13 +3,14 @@
 //
 // What bounds them: with random operands the card runs these contractions against its power
 // limit (the walk below alone: 2150 TFLOP/s on zeros, 1480-1510 on random bf16; the matrix
-// library 2120 and 1510), so the rate follows the energy per multiply-add, most of which past
+// library 2120 and 1510; Mixtral's gate/up call of 8192 tokens 2539 us on zeros, 3059 on random
+// data, at a clock of 1.75 GHz), so the rate follows the energy per multiply-add, most of which past
 // the matrix cores is LDS and cache traffic. A workgroup of 4 waves owns a 256-row x 256-token
 // output tile, alone on its CU, and each wave a 128 x 128 quarter of it with its accumulators
 // in 256 AGPRs: per K step of 128 bytes it reads 128 KB from LDS where 8 waves of 128 x 64 read
 // 192 KB (same loop, random bf16: 1500 against 1270 TFLOP/s) and the 256 x 128 tiles of
 // tiles.hip 192 KB plus 64 KB of register staging. Mixtral, 8192 tokens, 256 x 128 -> 256 x 256
-// tiles: gate/up 3607 -> 2943 us, down 1957 -> 1706 us (1310 and 1130 TFLOP/s).
+// tiles: gate/up 3607 -> 3060 us, down 1957 -> 1653 us (1257 and 1164 TFLOP/s; 2985 in another run).
 //
 // Both operands go straight into LDS (buffer_load ... lds, no registers), in two stages of
 // 64 KB. One step is two halves, the step's two 64-byte k-groups. While the 64 MFMAs of one half
@@ -384,7 +385,8 @@ __device__ __forceinline__ u32x4 join_tiles(const u32x2& a, const u32x2& b) {
 __device__ __forceinline__ int join_col(int lane) { return ((lane >> 4) & 1) * kRowTile + (lane >> 5) * 8; }
 
 // A copy of an accumulator, made here: without the assembly the compiler moved all of a wave's 256
-// accumulator registers to vector registers ahead of the branches of the epilogue, and spilled.
+// accumulator registers to vector registers ahead of the branches of the epilogue, and spilled 14
+// (DeepSeek-V2-Lite 2730 tokens down 189 -> 180 us without, Mixtral 8192 tokens 1707 -> 1692).
 __device__ __forceinline__ f32x4 acc_read(const f32x4& acc) {
   f32x4 v;
 #pragma unroll
@@ -534,7 +536,7 @@ __global__ __launch_bounds__(kXThreads, 1) void wide_gateup_kernel(ExpertArgs a)
 // times their routing weight (the combine's own rounding) and writes these terms at half the
 // bytes, which the combine only adds (per call, fp32 partials -> terms, down + combine:
 // DeepSeek-V2-Lite 2047 tokens 159 + 31 -> 153 + 20 us, Mixtral 8192 tokens 1742 + 122 -> 1716 +
-// 48). Rows past H (a multiple of 128) are clamped and not stored.
+// 48; since the epilogue no longer spills 146 + 20 and 1692 + 48). Rows past H (a multiple of 128) are clamped and not stored.
 template <int DT, bool kTerms>
 __global__ __launch_bounds__(kXThreads, 1) void wide_down_kernel(ExpertArgs a) {
   using S = typename Elem<DT>::S;

@@ -566,7 +566,8 @@ def run_tokens(args, wl, T, layers, L, dev, light=False):
             tflops = gateup_flops / (stage_us[1] * 1e-6) / 1e12
             peak = MFMA_BF16_PEAK_TFLOPS if dname == "bf16" else MFMA_FP32_PEAK_TFLOPS
             out["roofline"] = {
-                "kernel": "tile_gateup_kernel (W1/W3 x 128-token MFMA tiles + SiLU*up epilogue)",
+                "kernel": ("wide_gateup_kernel (W1/W3 x 256-token" if plan["wide_pairs"] else
+                           "tile_gateup_kernel (W1/W3 x 128-token") + " MFMA tiles + SiLU*up epilogue)",
                 "bound": "mfma",
                 "achieved": round(tflops, 1),
                 "peak": peak,
