@@ -96,13 +96,15 @@ def test_grouped_routing_block_graph(biased):
     _replays_match(run, out)
 
 
-def test_tiled_kernels_graph():
-    T, H, I, E, k = 1024, 256, 256, 8, 2
+@pytest.mark.parametrize("T,wide", [(1024, True), (480, False)])
+def test_tiled_kernels_graph(T, wide):
+    H, I, E, k = 256, 256, 8, 2
     x, logits, _ = _inputs(T, H, E, seed=40)
     pool, slots = make_pool(E, H, I, BF, seed=41)
     out = torch.empty_like(x)
     with tiled_min_tokens(0):
-        assert _lib.plan_info(T, H, I, E, k, _lib.SMX_BF16)["tiled"] == 1
+        plan = _lib.plan_info(T, H, I, E, k, _lib.SMX_BF16)
+        assert plan["tiled"] == 1 and (plan["wide_pairs"] > 0) == wide
         _replays_match(lambda: fused_moe_forward(x, logits, pool, slots, k, True, inplace=False), out)
 
 

@@ -65,7 +65,7 @@ IDENT = np.arange(E, dtype=np.int64)
 
 
 @pytest.mark.parametrize("T,k,tiled", [(1, 2, False), (4, 2, False), (32, 2, False),
-                                       (96, 3, False), (1024, 2, True)])
+                                       (96, 3, False), (1024, 2, True), (200, 2, True)])
 def test_routed_forward_reads_pages_past_4gib(big_pool, T, k, tiled):
     pool, slots, compact = big_pool
     x, logits = _inputs(T, seed=T + k)

@@ -29,7 +29,7 @@ def _check(y_clean, y_nan, bad):
     assert torch.isnan(y_nan[bad].float()).any()
 
 
-@pytest.mark.parametrize("T,tiled", [(1, False), (2, False), (32, False), (300, False), (1024, True)])
+@pytest.mark.parametrize("T,tiled", [(1, False), (2, False), (32, False), (300, False), (1024, True), (500, True)])
 def test_nan_token_stays_in_its_row(T, tiled):
     H, I, E, k = 256, 128, 8, 2
     x, logits, _ = _inputs(T, H, E, seed=T)

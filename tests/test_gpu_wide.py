@@ -10,8 +10,9 @@ import torch
 
 from oracle import moe_ref as ref
 from ae_amd import _lib
-from ae_amd.layers import (fused_moe_shared_forward, stack_fused_moe, stack_fused_moe_shared,
-                           tiled_min_tokens)
+from ae_amd.layers import (fused_moe_forward, fused_moe_shared_forward, stack_fused_moe,
+                           stack_fused_moe_shared, tiled_min_tokens)
+from ae_amd.layers._torch import ptr, stream_of
 from tests.helpers import (TOL, TORCH_TO_ORACLE, f32_of, make_pool, max_rel_err, nan_buffers,
                            to_oracle)
 
@@ -130,3 +131,23 @@ def test_wide_shared_expert(dtype, T, Is):
         to_oracle(x), f32_of(logits), to_oracle(pool), slots.cpu().numpy(), k, True, TORCH_TO_ORACLE[dtype],
         shared_page=to_oracle(page), shared_gate_logits=f32_of(sgate), routed_scaling_factor=1.0)
     assert max_rel_err(f32_of(y), y_ref) <= TOL[dtype]
+
+
+@pytest.mark.parametrize("I", [128, 1024])
+def test_wide_allocation_free_entry_gives_the_same_bits(I):
+    T, H, E, k = 700, 256, 4, 2
+    dtype = torch.float16
+    g = torch.Generator(device=DEV).manual_seed(I)
+    x = torch.randn((T, H), generator=g, device=DEV).to(dtype)
+    logits = (torch.randn((T, E), generator=g, device=DEV) * 2.0).to(dtype)
+    pool, slots = make_pool(E, H, I, dtype, num_slots=E + 1, seed=3)
+    y2 = torch.full_like(x, float("nan"))
+    w = torch.empty((T, k), dtype=torch.float32, device=DEV)
+    ids = torch.empty((T, k), dtype=torch.int32, device=DEV)
+    with tiled_min_tokens(0):
+        assert _lib.plan_info(T, H, I, E, k, _lib.SMX_F16)["wide_pairs"] > 0
+        y = fused_moe_forward(x.clone(), logits, pool, slots, k, True, inplace=False)
+        _lib.call("smx_fused_moe_forward_noalloc", ptr(x), ptr(y2), _lib.SMX_F16, T, H, ptr(logits), _lib.SMX_F16,
+                  E, k, 1, ptr(pool), pool.shape[0], pool.shape[1], ptr(slots), ptr(w), ptr(ids), stream_of(x))
+    torch.cuda.synchronize()
+    assert torch.equal(y, y2)
